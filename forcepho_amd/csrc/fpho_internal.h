@@ -74,6 +74,14 @@ FPHO_HDI int32_t order_key(float f) {
     return i >= 0 ? i : (i ^ 0x7FFFFFFF);
 }
 
+// The float of an order key.
+FPHO_HDI float key_float(int32_t k) {
+    k = k >= 0 ? k : (k ^ 0x7FFFFFFF);
+    float f;
+    __builtin_memcpy(&f, &k, 4);
+    return f;
+}
+
 // Everything the kernels need to know about one exposure of one patch.
 struct alignas(16) ExpDesc {
     const float *data, *ierr, *xpix, *ypix;  // patch pixel arrays
@@ -103,8 +111,10 @@ struct alignas(8) TileDesc {
     int32_t chunk0;    // first of the tile's 64-pixel slot boxes (plan-wide index)
     int64_t part_off;  // first float of this tile's gradient partials
     int32_t xlo, xhi, ylo, yhi;
+    float tmin;        // bright threshold: 0.1 sigma of its quietest pixel
+    int32_t flag;      // first flag word of the two-launch pixel pass
 };
-static_assert(sizeof(TileDesc) == 40, "TileDesc must be 40 bytes");
+static_assert(sizeof(TileDesc) == 48, "TileDesc must be 48 bytes");
 
 // One reduce output: band `band` of a patch, its tiles [tile0, tile0+ntiles)
 // are contiguous and their partials contiguous from part0 (stride n_src*7).
@@ -156,6 +166,12 @@ struct alignas(16) ImgGauss64 {
     double xcen, ycen, sfxx, sfyy, sfxy, hcs, ampA, pad0;
 };
 static_assert(sizeof(ImgGauss64) == 64, "ImgGauss64 must be 64 bytes");
+
+// Value parameters of ImgGauss alone: what the residual launch streams.
+struct alignas(16) HotGauss {
+    float xcen, ycen, sfxx, sfyy, sfxy, hcs, ampA, pad;
+};
+static_assert(sizeof(HotGauss) == 32, "HotGauss must be 32 bytes");
 
 // Precision modes of the pixel pass and reductions.
 enum Precision : int32_t {

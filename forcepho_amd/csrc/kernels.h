@@ -27,6 +27,14 @@ struct EvalArgs {
     int cull;              // skip Gaussians whose cutoff box misses the tile
     int mask_cap;          // Gaussians per exposure with an LDS slot mask (<= kMaskCapMax,
                            // a multiple of 8 so the activity words stay aligned)
+    // the two-launch pixel pass (n_items > 0)
+    const HotGauss *hot;     // [n_gauss]
+    const int2 *items;       // (tile, source or source count: chi2), in queue order
+    int64_t n_items;
+    uint64_t *flags;         // per tile [64 Gaussians][slot]: Gaussians with a
+                             // pixel inside the cutoff
+    double *resid;           // [slot][64] residual, slots as in slot_boxes
+    float *weight;           // [slot][64] -2 r ierr^2
     int act_words;         // 64-bit activity words per wave (<= kActWordsMax)
 };
 
@@ -44,12 +52,15 @@ struct SplineView {
 };
 
 hipError_t launch_convert(const ExpDesc *exps, int64_t n_exp, const fpho_source *props,
-                          ImgGauss *out, ImgGauss64 *out64, int4 *boxes, uint32_t *status,
-                          hipStream_t stream);
+                          ImgGauss *out, ImgGauss64 *out64, int4 *boxes, HotGauss *hot,
+                          uint32_t *status, hipStream_t stream);
 hipError_t launch_convert(const ExpDesc *exps, int64_t n_exp, const Source64 *props,
-                          ImgGauss *out, ImgGauss64 *out64, int4 *boxes, uint32_t *status,
-                          hipStream_t stream);
+                          ImgGauss *out, ImgGauss64 *out64, int4 *boxes, HotGauss *hot,
+                          uint32_t *status, hipStream_t stream);
 hipError_t launch_eval(const EvalArgs &a, hipStream_t stream);
+hipError_t launch_list_items(const TileDesc *tiles, const int32_t *queue, const ExpDesc *exps,
+                             const int32_t *start, int64_t n_tiles, int2 *items,
+                             hipStream_t stream);
 hipError_t launch_response(const double *dchi2, int32_t n_bands, int32_t n_src,
                            fpho_response *out, hipStream_t stream);
 hipError_t launch_reduce(const OutDesc *outs, int64_t n_outs, const float *gpart,

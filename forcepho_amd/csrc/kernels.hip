@@ -8,6 +8,9 @@
 //                       compute_gaussians_kernel.cu:262-301); one wave per
 //                       tile of 64*K pixels, no float atomics; LDS holds only
 //                       each wave's own slot masks and activity bits.
+//   residual_kernel, gradient_kernel<K>
+//                       the same in two launches, for small plans: one wave
+//                       per 64-pixel slot, then per (tile, source)
 //   reduce_kernel       fixed-order sum of tile partials (FP64 or FP32)
 //                       (replaces the shared-memory Accumulator,
 //                        compute_gaussians_kernel.cu:133-198)
@@ -165,7 +168,7 @@ template <typename Src>
 __global__ __launch_bounds__(128) void convert_kernel(
     const ExpDesc *__restrict__ exps, const Src *__restrict__ props,
     ImgGauss *__restrict__ out, ImgGauss64 *__restrict__ out64, int4 *__restrict__ boxes,
-    uint32_t *__restrict__ status) {
+    HotGauss *__restrict__ hot, uint32_t *__restrict__ status) {
     const ExpDesc e = exps[blockIdx.x];
     const int n = e.n_src * e.n_psf;
     for (int j = threadIdx.x; j < n; j += blockDim.x) {
@@ -178,6 +181,8 @@ __global__ __launch_bounds__(128) void convert_kernel(
         out[e.gauss_off + j] = g;
         out64[e.gauss_off + j] = g64;
         boxes[e.gauss_off + j] = make_int4(g.xlo, g.xhi, g.ylo, g.yhi);
+        if (hot)
+            hot[e.gauss_off + j] = {g.xcen, g.ycen, g.sfxx, g.sfyy, g.sfxy, g.hcs, g.ampA, 0.0f};
     }
 }
 
@@ -211,20 +216,135 @@ __device__ __forceinline__ bool boxed_out(int cull, const int4 gb, const int4 tb
 // polynomial (truncation 6e-16, amplified 1024-fold by the squarings to
 // < 1e-12 relative) -- two constants, so the rare FP64 path holds few
 // registers.
-__device__ __forceinline__ double pair_value64(const ImgGauss64 &g, float xp, float yp) {
+// Returns r - value (the subtraction fused with the last product).  The fused
+// forms are written out, here and in the pair functions below, so that every
+// kernel that evaluates a pair rounds it the same way.
+__device__ __forceinline__ double minus_value64(double r, const ImgGauss64 &g, float xp, float yp) {
     const double dx = (double)xp - g.xcen;
     const double dy = (double)yp - g.ycen;
-    const double vx = g.sfxx * dx + g.sfxy * dy;
-    const double vy = g.sfyy * dy + g.sfxy * dx;
-    const double ea = dx * vx + dy * vy;
+    const double vx = fma(g.sfxx, dx, g.sfxy * dy);
+    const double vy = fma(g.sfxy, dx, g.sfyy * dy);
+    const double ea = fma(dx, vx, dy * vy);
     const double n = __builtin_rint(ea);
     const double y = (ea - n) * (0.69314718055994530942 / 1024.0);
     double p = fma(y, fma(y, fma(y, 1.0 / 6.0, 0.5), 1.0), 1.0);
 #pragma unroll
     for (int j = 0; j < 10; ++j) p *= p;
     const double h = fma(vx, vx, fma(vy, vy, g.hcs));
-    return g.ampA * __builtin_ldexp(p, (int)n) * h;
+    return fma(-h, g.ampA * __builtin_ldexp(p, (int)n), r);
 }
+
+// Pass 1 of one pair: v' and the scaled exponent E' = s E.
+__device__ __forceinline__ float exponent1(float dx, float dy, float sfxx, float sfyy, float sfxy,
+                                           float &vx, float &vy) {
+    vx = fmaf(sfxx, dx, sfxy * dy);
+    vy = fmaf(sfyy, dy, sfxy * dx);
+    return fmaf(dx, vx, dy * vy);
+}
+
+// exp2(E') of a pair; a pair beyond the cutoff gives an exact zero.
+__device__ __forceinline__ float cut_exp(bool in, float ea) {
+    return __builtin_amdgcn_exp2f(in ? ea : -__builtin_huge_valf());
+}
+
+// c2 + (r^2 - d^2) ierr^2 of one pixel; rd holds an FP32 residual when the
+// residual is not kept in FP64.
+template <bool MIXED>
+__device__ __forceinline__ double add_chi2(double c2, double rd, float d, float ierr) {
+    if (MIXED) {
+        const double ie = (double)ierr, ds = (double)d * ie;
+        return fma(fma(rd, ie, -ds), fma(rd, ie, ds), c2);
+    }
+    const float rs = (float)rd * ierr;
+    const float ds = d * ierr;
+    return fma((double)rs - (double)ds, (double)rs + (double)ds, c2);
+}
+
+// The 12 pixel sums of one Gaussian that its derivatives are linear in.
+struct GradSums {
+    float PA = 0.f, X1 = 0.f, X2 = 0.f, Y1 = 0.f, Y2 = 0.f, Pxx = 0.f;
+    float Pyy = 0.f, Pxy = 0.f, Pe = 0.f, Peu = 0.f, Pea = 0.f, Pecr = 0.f;
+
+    // one pixel at offset (dx, dy) with rr = -2 r ierr^2
+    __device__ __forceinline__ void add(float dx, float dy, float rr, float sfxx, float sfyy,
+                                        float sfxy, float hcs) {
+        const float vx = fmaf(sfxx, dx, sfxy * dy);
+        const float vy = fmaf(sfyy, dy, sfxy * dx);
+        const float u = dx * vx;
+        const float ea = fmaf(dy, vy, u);
+        // a pixel beyond the cutoff gets gp = exp2(-inf) = 0, so all its
+        // terms below are exact zeros (every factor is finite)
+        const float gp = cut_exp(!(ea < kCutScaled), ea);
+        const float h = fmaf(vx, vx, fmaf(vy, vy, hcs));
+        const float ee = rr * gp;
+        const float a = ee * h;
+        PA = fmaf(ee, h, PA);
+        X1 = fmaf(a, vx, X1);
+        X2 = fmaf(ee, vx, X2);   // sum e v'x (s F applied in partials)
+        Y1 = fmaf(a, vy, Y1);
+        Y2 = fmaf(ee, vy, Y2);   // sum e v'y
+        const float ax = a * dx;
+        const float ay = a * dy;
+        Pxx = fmaf(ax, dx, Pxx);
+        Pxy = fmaf(ax, dy, Pxy);
+        Pyy = fmaf(ay, dy, Pyy);
+        Pe = fmaf(rr, gp, Pe);
+        Peu = fmaf(ee, u, Peu);
+        Pea = fmaf(ee, ea, Pea);
+        Pecr = fmaf(ee, fmaf(dy, vx, dx * vy), Pecr);
+    }
+};
+
+// A source's 7 partials over the pixels of one lane (position in pixels).
+struct SourcePartials {
+    float p0 = 0.f, sx = 0.f, sy = 0.f, p3 = 0.f, p4 = 0.f, p5 = 0.f, p6 = 0.f;
+
+    // per-Gaussian epilogue: image-space derivative sums -> 7 partials
+    __device__ __forceinline__ void add(const ImgGauss &G, const GradSums &q) {
+        const float ke = G.k_e * q.Pe;
+        const float gfx = fmaf(G.k_u, q.Peu, fmaf(G.k_axx, q.Pxx, ke));
+        const float gfy = fmaf(G.k_u, q.Pea - q.Peu, fmaf(G.k_axx, q.Pyy, ke));
+        const float gfxy = fmaf(G.k_u, q.Pecr, G.k_axy * q.Pxy);
+        p0 = fmaf(G.cA_flux, q.PA, p0);
+        p5 = fmaf(G.cA_n, q.PA, p5);
+        p6 = fmaf(G.cA_rh, q.PA, p6);
+        p3 = fmaf(G.cA_q, q.PA, p3);
+        p3 = fmaf(G.dFxx_dQ, gfx, p3);
+        p3 = fmaf(G.dFyy_dQ, gfy, p3);
+        p3 = fmaf(G.dFxy_dQ, gfxy, p3);
+        p4 = fmaf(G.cA_pa, q.PA, p4);
+        p4 = fmaf(G.dFxx_dPA, gfx, p4);
+        p4 = fmaf(G.dFyy_dPA, gfy, p4);
+        p4 = fmaf(G.dFxy_dPA, gfxy, p4);
+        // sum e (sF v')_x = sfxx sum e v'x + sfxy sum e v'y (and for y)
+        const float fX = fmaf(G.sfxx, q.X2, G.sfxy * q.Y2);
+        const float fY = fmaf(G.sfxy, q.X2, G.sfyy * q.Y2);
+        sx = fmaf(G.k_x1, q.X1, fmaf(G.k_x2, fX, sx));
+        sy = fmaf(G.k_x1, q.Y1, fmaf(G.k_x2, fY, sy));
+    }
+
+    // sum over the wave and write (lane 0); the sky-position derivatives
+    // share the source's CW matrix
+    __device__ __forceinline__ void write(float *__restrict__ o, const float *__restrict__ CW,
+                                          int lane) {
+        p0 = wave_sum(p0);
+        sx = wave_sum(sx);
+        sy = wave_sum(sy);
+        p3 = wave_sum(p3);
+        p4 = wave_sum(p4);
+        p5 = wave_sum(p5);
+        p6 = wave_sum(p6);
+        if (lane == 0) {
+            o[0] = p0;
+            o[1] = fmaf(CW[0], sx, CW[2] * sy);  // dx/dalpha, dy/dalpha
+            o[2] = fmaf(CW[1], sx, CW[3] * sy);  // dx/ddelta, dy/ddelta
+            o[3] = p3;
+            o[4] = p4;
+            o[5] = p5;
+            o[6] = p6;
+        }
+    }
+};
 
 // Evaluate one wave tile.  `tile` must be wave-uniform (an SGPR value) so
 // every descriptor and Gaussian record load below is a scalar load (the
@@ -366,15 +486,14 @@ __device__ __forceinline__ void eval_tile(int tile, const TileDesc *__restrict__
                     dx -= xcl;
                     dy -= ycl;
                 }
-                const float vx = sfxx * dx + sfxy * dy;
-                const float vy = sfyy * dy + sfxy * dx;
-                const float ea = dx * vx + dy * vy;      // s E
+                float vx, vy;
+                const float ea = exponent1(dx, dy, sfxx, sfyy, sfxy, vx, vy);   // s E
                 const bool in = !(ea < kCutScaled);       // E <= 36 (cutoff)
                 if (__builtin_amdgcn_ballot_w64(in) == 0) continue;
                 m |= 1u << k;
                 {
                     // a lane beyond the cutoff adds an exact zero
-                    const float gp = __builtin_amdgcn_exp2f(in ? ea : -__builtin_huge_valf());
+                    const float gp = cut_exp(in, ea);
                     const float h = fmaf(vx, vx, fmaf(vy, vy, hcs));
                     const float c = ampA * gp * h;
                     if (MIXED) {
@@ -384,7 +503,7 @@ __device__ __forceinline__ void eval_tile(int tile, const TileDesc *__restrict__
                             // loop they would hold 4K more registers)
                             float xk = x[k], yk = y[k];
                             asm volatile("" : "+v"(xk), "+v"(yk));
-                            rd[k] -= pair_value64(g64[i], xk, yk);
+                            rd[k] = minus_value64(rd[k], g64[i], xk, yk);
                         } else
                             rd[k] -= (double)c;
                     } else {
@@ -417,18 +536,8 @@ __device__ __forceinline__ void eval_tile(int tile, const TileDesc *__restrict__
             dk = e.data[t.pix0 + p];
             iek = e.ierr[t.pix0 + p];
         }
-        if (MIXED) {
-            r[k] = (float)rd[k];
-            const double rs = rd[k] * (double)iek;
-            const double ds = (double)dk * (double)iek;
-            c2 += (rs - ds) * (rs + ds);
-        } else {
-            const float rs = r[k] * iek;
-            const float ds = dk * iek;
-            double c = (double)rs - (double)ds;
-            c *= (double)rs + (double)ds;
-            c2 += c;
-        }
+        if (MIXED) r[k] = (float)rd[k];
+        c2 = add_chi2<MIXED>(c2, MIXED ? rd[k] : (double)r[k], dk, iek);
         if (e.residual != nullptr && p < t.npix) e.residual[t.pix0 + p] = r[k];
         rr[k] = -2.0f * ((r[k] * iek) * iek);  // -2 r ierr^2
         // finish this slot here: deferred, its loaded values would spill
@@ -440,7 +549,7 @@ __device__ __forceinline__ void eval_tile(int tile, const TileDesc *__restrict__
     // ---- pass 2: per source, 7 partials   (common_kernel.cc:95-143)
     float *__restrict__ out = gpart + t.part_off;
     for (int s = 0; s < n_src; ++s) {
-        float p0 = 0.f, sx = 0.f, sy = 0.f, p3 = 0.f, p4 = 0.f, p5 = 0.f, p6 = 0.f;
+        SourcePartials src;
         const int i0 = s * n_psf;
         bool touched = false;
         for (int w = i0 / kWave; w <= (i0 + n_psf - 1) / kWave; ++w) {
@@ -464,9 +573,7 @@ __device__ __forceinline__ void eval_tile(int tile, const TileDesc *__restrict__
             const float xc = G.xcen, yc = G.ycen;
             const float xcl = CENTRE ? G.xcen_lo : 0.0f, ycl = CENTRE ? G.ycen_lo : 0.0f;
             const float sfxx = G.sfxx, sfyy = G.sfyy, sfxy = G.sfxy, hcs = G.hcs;
-            // the 12 per-Gaussian pixel sums (over this lane's K pixels)
-            float PA = 0.f, X1 = 0.f, X2 = 0.f, Y1 = 0.f, Y2 = 0.f, Pxx = 0.f;
-            float Pyy = 0.f, Pxy = 0.f, Pe = 0.f, Peu = 0.f, Pea = 0.f, Pecr = 0.f;
+            GradSums q;   // over this lane's K pixels
 #pragma unroll
             for (int k = 0; k < K; ++k) {
                 if (!(m & (1u << k))) continue;
@@ -476,52 +583,9 @@ __device__ __forceinline__ void eval_tile(int tile, const TileDesc *__restrict__
                     dx -= xcl;
                     dy -= ycl;
                 }
-                const float vx = sfxx * dx + sfxy * dy;
-                const float vy = sfyy * dy + sfxy * dx;
-                const float u = dx * vx;
-                const float ea = fmaf(dy, vy, u);
-                // a pixel beyond the cutoff gets gp = exp2(-inf) = 0, so all
-                // its terms below are exact zeros (every factor is finite)
-                const bool in = !(ea < kCutScaled);
-                const float gp = __builtin_amdgcn_exp2f(in ? ea : -__builtin_huge_valf());
-                const float h = fmaf(vx, vx, fmaf(vy, vy, hcs));
-                const float ee = rr[k] * gp;
-                const float a = ee * h;
-                PA += a;
-                X1 = fmaf(a, vx, X1);
-                X2 = fmaf(ee, vx, X2);   // sum e v'x (s F applied below)
-                Y1 = fmaf(a, vy, Y1);
-                Y2 = fmaf(ee, vy, Y2);   // sum e v'y
-                const float ax = a * dx;
-                const float ay = a * dy;
-                Pxx = fmaf(ax, dx, Pxx);
-                Pxy = fmaf(ax, dy, Pxy);
-                Pyy = fmaf(ay, dy, Pyy);
-                Pe += ee;
-                Peu = fmaf(ee, u, Peu);
-                Pea = fmaf(ee, ea, Pea);
-                Pecr = fmaf(ee, fmaf(dy, vx, dx * vy), Pecr);
+                q.add(dx, dy, rr[k], sfxx, sfyy, sfxy, hcs);
             }
-            // per-Gaussian epilogue: image-space derivative sums -> 7 partials
-            const float gfx = G.k_axx * Pxx + G.k_e * Pe + G.k_u * Peu;
-            const float gfy = G.k_axx * Pyy + G.k_e * Pe + G.k_u * (Pea - Peu);
-            const float gfxy = G.k_axy * Pxy + G.k_u * Pecr;
-            p0 = fmaf(G.cA_flux, PA, p0);
-            p5 = fmaf(G.cA_n, PA, p5);
-            p6 = fmaf(G.cA_rh, PA, p6);
-            p3 = fmaf(G.cA_q, PA, p3);
-            p3 = fmaf(G.dFxx_dQ, gfx, p3);
-            p3 = fmaf(G.dFyy_dQ, gfy, p3);
-            p3 = fmaf(G.dFxy_dQ, gfxy, p3);
-            p4 = fmaf(G.cA_pa, PA, p4);
-            p4 = fmaf(G.dFxx_dPA, gfx, p4);
-            p4 = fmaf(G.dFyy_dPA, gfy, p4);
-            p4 = fmaf(G.dFxy_dPA, gfxy, p4);
-            // sum e (sF v')_x = sfxx sum e v'x + sfxy sum e v'y (and for y)
-            const float fX = sfxx * X2 + sfxy * Y2;
-            const float fY = sfyy * Y2 + sfxy * X2;
-            sx = fmaf(G.k_x1, X1, fmaf(G.k_x2, fX, sx));
-            sy = fmaf(G.k_x1, Y1, fmaf(G.k_x2, fY, sy));
+            src.add(G, q);
           }
         }
         float *o = out + kNParams * s;
@@ -530,24 +594,7 @@ __device__ __forceinline__ void eval_tile(int tile, const TileDesc *__restrict__
             if (lane < kNParams) o[lane] = 0.0f;
             continue;
         }
-        p0 = wave_sum(p0);
-        sx = wave_sum(sx);
-        sy = wave_sum(sy);
-        p3 = wave_sum(p3);
-        p4 = wave_sum(p4);
-        p5 = wave_sum(p5);
-        p6 = wave_sum(p6);
-        if (lane == 0) {
-            // the sky-position derivatives share the source's CW matrix
-            const float *CW = e.CW + 4 * s;
-            o[0] = p0;
-            o[1] = CW[0] * sx + CW[2] * sy;  // dx/dalpha, dy/dalpha
-            o[2] = CW[1] * sx + CW[3] * sy;  // dx/ddelta, dy/ddelta
-            o[3] = p3;
-            o[4] = p4;
-            o[5] = p5;
-            o[6] = p6;
-        }
+        src.write(o, e.CW + 4 * s, lane);
     }
 }
 
@@ -622,6 +669,333 @@ __global__ __launch_bounds__(256) FPHO_EVAL_OCCUPANCY void eval_persistent_kerne
                             reinterpret_cast<uint64_t *>(lds_mask + W * mask_cap) +
                                 w * act_words, act_words);
     }
+}
+
+// ------------------------------------------------ pixel pass in two launches
+//
+// For plans whose tiles do not fill the chip (two_launches() in runtime.hip):
+// residual_kernel runs one wave per 64-pixel slot, gradient_kernel one wave
+// per (tile, source), so a tile's work is spread over its slots and then over
+// its sources instead of being one wave's.  A pixel's Gaussians are still
+// subtracted in index order by one lane, a source's partials are still summed
+// over the tile's K slots by one wave, and pass 2 visits the slots that pass
+// 1 found active, so every result is eval_tile's bit for bit.
+//
+// What bounds it: VALU issue, and on small plans the serial chain of the
+// heaviest wave.  Measured (us, one wave per tile -> two launches): 16 tiles
+// of 54 Gaussians 58 -> 33; 2048 tiles of 720 535 -> 311; 6144 tiles of 2160
+// 1440 -> 1206; 575 tiles of up to 1620 (four patches) 882 -> 158.
+
+// A pointer known to be to device memory (descriptors hold generic ones), so
+// loads take a scalar base and a 32-bit lane offset.
+template <typename T>
+using Global = const T __attribute__((address_space(1))) *;
+template <typename T>
+__device__ __forceinline__ Global<T> global(const T *p) {
+    return (Global<T>)p;
+}
+
+// False only if no point of the box [xlo, xhi] x [ylo, yhi] (relative to the
+// Gaussian's centre) lies inside its cutoff ellipse E <= 36.  The smallest E
+// of a box that does not hold the centre is on an edge that faces the centre;
+// along such an edge E is a parabola with its minimum at -(Fxy / Fyy) dx (or
+// its twin).  sF is negative, so the smallest E is the largest E'.  The limit
+// is widened by 0.1% and by the FP32 error of E, 4e-6 of it per 1 / (1 -
+// rho^2), here and in pass 1; a NaN or an indefinite F counts as meeting.
+__device__ __forceinline__ bool meets(float xlo, float xhi, float ylo, float yhi, float sfxx,
+                                      float sfyy, float sfxy) {
+    const float dx = __builtin_amdgcn_fmed3f(0.0f, xlo, xhi);
+    const float dy = __builtin_amdgcn_fmed3f(0.0f, ylo, yhi);
+    const float ya = __builtin_amdgcn_fmed3f(-sfxy * __builtin_amdgcn_rcpf(sfyy) * dx, ylo, yhi);
+    const float xb = __builtin_amdgcn_fmed3f(-sfxy * __builtin_amdgcn_rcpf(sfxx) * dy, xlo, xhi);
+    const float ea = fmaf(dx, fmaf(sfxx, dx, 2.0f * sfxy * ya), sfyy * ya * ya);
+    const float eb = fmaf(dy, fmaf(sfyy, dy, 2.0f * sfxy * xb), sfxx * xb * xb);
+    const float k = sfxx * sfyy;
+    const float wide = k * __builtin_amdgcn_rcpf(fmaxf(fmaf(-sfxy, sfxy, k), 0.0f));
+    return !(fmaxf(ea, eb) < kCutScaled * fmaf(4e-6f, wide, 1.001f));
+}
+
+// Set bits of m below this lane.
+__device__ __forceinline__ int rank_in(uint64_t m) {
+    return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
+                                     __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0));
+}
+
+// Lane values in the order "lanes set in m first" (a permutation of the wave).
+__device__ __forceinline__ uint32_t set_first(uint64_t m, bool set, int lane, uint32_t v) {
+    const int rank = rank_in(m);
+    const int to = set ? rank : __builtin_popcountll(m) + lane - rank;
+    return (uint32_t)__builtin_amdgcn_ds_permute(to << 2, (int)v);
+}
+
+// Pass 1 of one slot.  Each block of 64 Gaussians is tested at once (lane j:
+// Gaussian base + j) and the ones that meet the slot are listed in a vector
+// register as record offsets, so a visit costs a readlane and a scalar load.
+// kVisits of them go through together: one wait for their records and one
+// test for bright terms (four small patches: 218 us a pass with four at once,
+// 232 with two; eight records do not fit the scalar registers).
+template <int K, bool MIXED, bool CENTRE>
+__global__ __launch_bounds__(kWave) FPHO_EVAL_OCCUPANCY void residual_kernel(
+    const TileDesc *__restrict__ tiles, const int32_t *__restrict__ queue,
+    const ExpDesc *__restrict__ exps, const ImgGauss *__restrict__ gauss,
+    const ImgGauss64 *__restrict__ gauss64, const HotGauss *__restrict__ hot,
+    const int4 *__restrict__ slot_boxes, uint64_t *__restrict__ flags,
+    double *__restrict__ resid, float *__restrict__ weight, int32_t cull) {
+    constexpr int kVisits = 4;
+    const int lane = threadIdx.x;
+    const int wave = xcd_swizzle<kXcdChunk>((int)blockIdx.x, (int)gridDim.x);
+    const TileDesc t = tiles[queue[wave / K]];
+    const int k = wave % K;
+    const int npix = t.npix - k * kWave;   // of this slot and the ones after it
+    if (npix <= 0) return;
+    const int pix0 = t.pix0 + k * kWave;
+    const ExpDesc &e = exps[t.exp];
+    const int4 box = slot_boxes[t.chunk0 + k];
+    // 0.01 pixel covers the FP32 rounding of the centre
+    const float xlo = key_float(box.x) - 0.01f, xhi = key_float(box.y) + 0.01f;
+    const float ylo = key_float(box.z) - 0.01f, yhi = key_float(box.w) + 0.01f;
+    const ImgGauss *__restrict__ g = gauss + e.gauss_off;
+    const ImgGauss64 *__restrict__ g64 = gauss64 + e.gauss_off;
+    const char *__restrict__ gh = reinterpret_cast<const char *>(hot + e.gauss_off);
+    const Global<HotGauss> gv = global(hot + e.gauss_off);
+    const int ng = e.n_src * e.n_psf;
+
+    float x = kMaskedCoord, y = kMaskedCoord, r = 0.0f, iek = 0.0f;
+    if (lane < npix) {
+        x = global(e.xpix + pix0)[(uint32_t)lane] - e.x0;
+        y = global(e.ypix + pix0)[(uint32_t)lane] - e.y0;
+        r = global(e.data + pix0)[(uint32_t)lane];
+        iek = global(e.ierr + pix0)[(uint32_t)lane];
+    }
+    double rd = (double)r;
+
+    // pass 1 of one visit: the term, and whether a lane is inside the cutoff
+    auto term = [&](const HotGauss &H, float xl, float yl, uint64_t &in_lanes) {
+        float dx = x - H.xcen, dy = y - H.ycen, vx, vy;
+        if (CENTRE) {   // the pixel offset from the FP64 centre
+            dx -= xl;
+            dy -= yl;
+        }
+        const float ea = exponent1(dx, dy, H.sfxx, H.sfyy, H.sfxy, vx, vy);
+        const bool in = !(ea < kCutScaled);
+        in_lanes = __builtin_amdgcn_ballot_w64(in);
+        const float gp = cut_exp(in, ea);
+        return H.ampA * gp * fmaf(vx, vx, fmaf(vy, vy, H.hcs));
+    };
+    auto subtract_bright = [&](float c, uint32_t off) {
+        if (__builtin_amdgcn_ballot_w64(fabsf(c) > t.tmin) == 0) {
+            rd -= (double)c;
+            return;
+        }
+        // FP64 copies of the coordinates made here: kept across the loop they
+        // would hold 4 more registers
+        float xb = x, yb = y;
+        asm volatile("" : "+v"(xb), "+v"(yb));
+        const double b = minus_value64(rd, g64[off / sizeof(HotGauss)], xb, yb);
+        rd = fabsf(c) > t.tmin ? b : rd - (double)c;
+    };
+
+    float hx, hy, hxx, hyy, hxy;   // lane j: Gaussian base + j
+    auto fetch = [&](int j) {
+        const Global<HotGauss> p = gv + (uint32_t)min(j, ng - 1);
+        hx = p->xcen;
+        hy = p->ycen;
+        hxx = p->sfxx;
+        hyy = p->sfyy;
+        hxy = p->sfxy;
+    };
+    fetch(lane);
+    uint64_t *__restrict__ fl = flags + t.flag + k;
+    for (int base = 0; base < ng; base += kWave, fl += K) {
+        const int j = base + lane;
+        const bool hit =
+            j < ng && (cull == 0 || meets(xlo - hx, xhi - hx, ylo - hy, yhi - hy, hxx, hyy, hxy));
+        fetch(j + kWave);   // the next block's, under this block's visits
+        const uint64_t m = __builtin_amdgcn_ballot_w64(hit);
+        const int cnt = __builtin_popcountll(m);
+        const uint32_t list = set_first(
+            m, hit, lane, (uint32_t)min(j, ng - 1) * (uint32_t)sizeof(HotGauss));
+        // bit cnt - 1 - n of act: the n-th visit had a lane inside the cutoff
+        // (shifted in through the scalar carry: two additions of act to itself)
+        uint32_t act_lo = 0, act_hi = 0;
+        auto note = [&](uint64_t in_lanes) {
+            asm("s_cmp_lg_u64 %2, 0\n\ts_addc_u32 %0, %0, %0\n\ts_addc_u32 %1, %1, %1"
+                : "+s"(act_lo), "+s"(act_hi)
+                : "s"(in_lanes)
+                : "scc");
+        };
+        int n = 0;
+        for (; n + kVisits <= cnt; n += kVisits) {
+            uint32_t off[kVisits];
+            HotGauss H[kVisits];
+            float xl[kVisits], yl[kVisits], c[kVisits], top = 0.0f;
+#pragma unroll
+            for (int u = 0; u < kVisits; ++u) off[u] = __builtin_amdgcn_readlane(list, n + u);
+#pragma unroll
+            for (int u = 0; u < kVisits; ++u) {
+                H[u] = *reinterpret_cast<const HotGauss *>(gh + off[u]);
+                if (CENTRE) {
+                    xl[u] = g[off[u] / sizeof(HotGauss)].xcen_lo;
+                    yl[u] = g[off[u] / sizeof(HotGauss)].ycen_lo;
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);   // all loads before the first wait
+#pragma unroll
+            for (int u = 0; u < kVisits; ++u) {
+                uint64_t in_lanes;
+                c[u] = term(H[u], CENTRE ? xl[u] : 0.0f, CENTRE ? yl[u] : 0.0f, in_lanes);
+                note(in_lanes);
+                if (MIXED) top = fmaxf(top, fabsf(c[u]));
+            }
+            if (!MIXED) {
+#pragma unroll
+                for (int u = 0; u < kVisits; ++u) r -= c[u];
+            } else if (__builtin_amdgcn_ballot_w64(top > t.tmin) == 0) {
+#pragma unroll
+                for (int u = 0; u < kVisits; ++u) rd -= (double)c[u];
+            } else {
+#pragma unroll
+                for (int u = 0; u < kVisits; ++u) subtract_bright(c[u], off[u]);
+            }
+        }
+        for (; n < cnt; ++n) {
+            const uint32_t off = __builtin_amdgcn_readlane(list, n);
+            const ImgGauss &G = g[off / sizeof(HotGauss)];
+            uint64_t in_lanes;
+            const float c = term(*reinterpret_cast<const HotGauss *>(gh + off),
+                                 CENTRE ? G.xcen_lo : 0.0f, CENTRE ? G.ycen_lo : 0.0f, in_lanes);
+            note(in_lanes);
+            if (MIXED)
+                subtract_bright(c, off);
+            else
+                r -= c;
+        }
+        const uint64_t act = (uint64_t)act_hi << 32 | act_lo;
+        const uint64_t word = __builtin_amdgcn_ballot_w64(
+            hit && ((act >> ((cnt - 1 - rank_in(m)) & 63)) & 1));
+        if (lane == 0) *fl = word;
+    }
+    if (!MIXED) rd = (double)r;
+    r = (float)rd;
+    const uint32_t o = (uint32_t)(t.chunk0 + k) * kWave + lane;
+    resid[o] = rd;
+    weight[o] = -2.0f * ((r * iek) * iek);   // -2 r ierr^2
+    if (e.residual != nullptr && lane < npix) e.residual[pix0 + lane] = r;
+}
+
+// Pass 2 of one source of one tile, or (source n_src) the tile's chi2.
+template <int K, bool MIXED, bool CENTRE>
+__global__ __launch_bounds__(kWave) FPHO_EVAL_OCCUPANCY void gradient_kernel(
+    const TileDesc *__restrict__ tiles, const int2 *__restrict__ items,
+    const ExpDesc *__restrict__ exps, const ImgGauss *__restrict__ gauss,
+    const uint64_t *__restrict__ flags, const double *__restrict__ resid,
+    const float *__restrict__ weight, float *__restrict__ gpart, double *__restrict__ cpart) {
+    const int lane = threadIdx.x;
+    const int2 item = items[xcd_swizzle<kXcdChunk>((int)blockIdx.x, (int)gridDim.x)];
+    const int tile = item.x, s = item.y;
+    const TileDesc t = tiles[tile];
+    const ExpDesc &e = exps[t.exp];
+    const uint32_t slot = (uint32_t)t.chunk0 * kWave;
+    if (s == e.n_src) {
+        // sum (r^2 - d^2) ierr^2 (compute_gaussians_kernel.cu:276-287)
+        double c2 = 0.0;
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            const uint32_t p = k * kWave + lane;
+            float dk = 0.0f, iek = 0.0f;
+            double rd = 0.0;
+            if ((int)p < t.npix) {
+                dk = global(e.data + t.pix0)[p];
+                iek = global(e.ierr + t.pix0)[p];
+                rd = resid[slot + p];
+            }
+            c2 = add_chi2<MIXED>(c2, rd, dk, iek);
+        }
+        c2 = wave_sum(c2);
+        if (lane == 0) cpart[tile] = c2;
+        return;
+    }
+    float x[K], y[K], rr[K];
+    if (t.npix == K * kWave) {
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            const uint32_t p = k * kWave + lane;
+            x[k] = global(e.xpix + t.pix0)[p] - e.x0;
+            y[k] = global(e.ypix + t.pix0)[p] - e.y0;
+            rr[k] = (weight + slot)[p];
+        }
+    } else {
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            const uint32_t p = k * kWave + lane;
+            x[k] = y[k] = kMaskedCoord;
+            rr[k] = 0.0f;
+            if ((int)p < t.npix) {
+                x[k] = global(e.xpix + t.pix0)[p] - e.x0;
+                y[k] = global(e.ypix + t.pix0)[p] - e.y0;
+                rr[k] = (weight + slot)[p];
+            }
+        }
+    }
+    const ImgGauss *__restrict__ g = gauss + e.gauss_off;
+    const uint32_t *__restrict__ fl = reinterpret_cast<const uint32_t *>(flags + t.flag);
+    const int n_psf = e.n_psf;
+    SourcePartials src;
+    bool touched = false;
+    for (int cb = 0; cb < n_psf; cb += kWave) {
+        // lane l: the slots in which Gaussian i is active
+        const bool valid = cb + lane < n_psf;
+        const uint32_t i = s * n_psf + (valid ? cb + lane : 0);
+        uint32_t mask = 0;
+        if (valid) {
+            const uint32_t f = (i >> 6) * (2 * K) + ((i >> 5) & 1);
+#pragma unroll
+            for (int k = 0; k < K; ++k)
+                if (k * kWave < t.npix) mask |= ((fl[f + 2 * k] >> (i & 31)) & 1) << k;
+        }
+        const uint64_t m = __builtin_amdgcn_ballot_w64(mask != 0);
+        const int cnt = __builtin_popcountll(m);
+        if (cnt == 0) continue;
+        touched = true;
+        const uint32_t list = set_first(m, mask != 0, lane, i << 8 | mask);
+        for (int n = 0; n < cnt; ++n) {
+            const uint32_t v = __builtin_amdgcn_readlane(list, n);
+            const ImgGauss &G = g[v >> 8];
+            // read once: left to the slots, each would load them again
+            const float xc = G.xcen, yc = G.ycen;
+            const float xcl = CENTRE ? G.xcen_lo : 0.0f, ycl = CENTRE ? G.ycen_lo : 0.0f;
+            const float sfxx = G.sfxx, sfyy = G.sfyy, sfxy = G.sfxy, hcs = G.hcs;
+            GradSums q;
+#pragma unroll
+            for (int k = 0; k < K; ++k) {
+                if (!(v & (1u << k))) continue;
+                float dx = x[k] - xc, dy = y[k] - yc;
+                if (CENTRE) {
+                    dx -= xcl;
+                    dy -= ycl;
+                }
+                q.add(dx, dy, rr[k], sfxx, sfyy, sfxy, hcs);
+            }
+            src.add(G, q);
+        }
+    }
+    float *o = gpart + t.part_off + kNParams * s;
+    if (touched)
+        src.write(o, e.CW + 4 * s, lane);
+    else if (lane < kNParams)
+        o[lane] = 0.0f;
+}
+
+// The gradient launch's waves: for the q-th tile of the queue, its sources
+// and then its chi2, from items[start[q]].
+__global__ __launch_bounds__(256) void list_items_kernel(
+    const TileDesc *__restrict__ tiles, const int32_t *__restrict__ queue,
+    const ExpDesc *__restrict__ exps, const int32_t *__restrict__ start, int32_t n_tiles,
+    int2 *__restrict__ items) {
+    const int q = blockIdx.x * blockDim.x + threadIdx.x;
+    if (q >= n_tiles) return;
+    const int tile = queue[q], n_src = exps[tiles[tile].exp].n_src;
+    for (int s = 0; s <= n_src; ++s) items[start[q] + s] = make_int2(tile, s);
 }
 
 __global__ void zero_counter_kernel(int32_t *counter) {
@@ -871,24 +1245,24 @@ __global__ __launch_bounds__(256) void response_kernel(const double *__restrict_
 
 template <typename Src>
 static hipError_t launch_convert_t(const ExpDesc *exps, int64_t n_exp, const Src *props,
-                                   ImgGauss *out, ImgGauss64 *out64, int4 *boxes,
+                                   ImgGauss *out, ImgGauss64 *out64, int4 *boxes, HotGauss *hot,
                                    uint32_t *status, hipStream_t stream) {
     if (n_exp <= 0) return hipSuccess;
     hipLaunchKernelGGL(convert_kernel<Src>, dim3((unsigned)n_exp), dim3(128), 0, stream,
-                       exps, props, out, out64, boxes, status);
+                       exps, props, out, out64, boxes, hot, status);
     return hipGetLastError();
 }
 
 hipError_t launch_convert(const ExpDesc *exps, int64_t n_exp, const fpho_source *props,
-                          ImgGauss *out, ImgGauss64 *out64, int4 *boxes, uint32_t *status,
-                          hipStream_t stream) {
-    return launch_convert_t(exps, n_exp, props, out, out64, boxes, status, stream);
+                          ImgGauss *out, ImgGauss64 *out64, int4 *boxes, HotGauss *hot,
+                          uint32_t *status, hipStream_t stream) {
+    return launch_convert_t(exps, n_exp, props, out, out64, boxes, hot, status, stream);
 }
 
 hipError_t launch_convert(const ExpDesc *exps, int64_t n_exp, const Source64 *props,
-                          ImgGauss *out, ImgGauss64 *out64, int4 *boxes, uint32_t *status,
-                          hipStream_t stream) {
-    return launch_convert_t(exps, n_exp, props, out, out64, boxes, status, stream);
+                          ImgGauss *out, ImgGauss64 *out64, int4 *boxes, HotGauss *hot,
+                          uint32_t *status, hipStream_t stream) {
+    return launch_convert_t(exps, n_exp, props, out, out64, boxes, hot, status, stream);
 }
 
 hipError_t launch_response(const double *dchi2, int32_t n_bands, int32_t n_src,
@@ -901,6 +1275,15 @@ hipError_t launch_response(const double *dchi2, int32_t n_bands, int32_t n_src,
 
 template <int K, bool MIXED, bool CENTRE>
 static hipError_t launch_eval_k(const EvalArgs &a, hipStream_t stream) {
+    if (a.n_items > 0) {
+        hipLaunchKernelGGL((residual_kernel<K, MIXED, CENTRE>), dim3((unsigned)(K * a.n_tiles)),
+                           dim3(kWave), 0, stream, a.tiles, a.queue, a.exps, a.gauss, a.gauss64,
+                           a.hot, a.slot_boxes, a.flags, a.resid, a.weight, (int32_t)a.cull);
+        hipLaunchKernelGGL((gradient_kernel<K, MIXED, CENTRE>), dim3((unsigned)a.n_items),
+                           dim3(kWave), 0, stream, a.tiles, a.items, a.exps, a.gauss, a.flags,
+                           a.resid, a.weight, a.gpart, a.cpart);
+        return hipGetLastError();
+    }
     const int W = a.waves_per_group;
     // per wave: the slot mask bytes, then the activity words
     const size_t lds = (size_t)W * ((size_t)a.mask_cap + 8 * (size_t)a.act_words);
@@ -938,6 +1321,15 @@ hipError_t launch_eval(const EvalArgs &a, hipStream_t stream) {
         case kPrecMixedCentre: return launch_eval_p<true, true>(a, stream);
         default: return launch_eval_p<false, false>(a, stream);
     }
+}
+
+hipError_t launch_list_items(const TileDesc *tiles, const int32_t *queue, const ExpDesc *exps,
+                             const int32_t *start, int64_t n_tiles, int2 *items,
+                             hipStream_t stream) {
+    if (n_tiles <= 0) return hipSuccess;
+    hipLaunchKernelGGL(list_items_kernel, dim3((unsigned)((n_tiles + 255) / 256)), dim3(256), 0,
+                       stream, tiles, queue, exps, start, (int32_t)n_tiles, items);
+    return hipGetLastError();
 }
 
 hipError_t launch_reduce(const OutDesc *outs, int64_t n_outs, const float *gpart,

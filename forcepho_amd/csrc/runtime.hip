@@ -159,6 +159,12 @@ struct Plan {
     DevVec<ImgGauss> gauss;
     DevVec<ImgGauss64> gauss64;
     DevVec<int4> gboxes;
+    // two-launch pixel pass (empty unless the plan uses it)
+    DevVec<HotGauss> hot;
+    DevVec<int2> items;
+    DevVec<uint64_t> flags;
+    DevVec<double> resid;
+    DevVec<float> weight;
     DevVec<int4> slot_boxes;
     DevVec<float> gpart;
     DevVec<double> cpart;
@@ -196,6 +202,7 @@ struct fpho_patch {
     // at the exposure start): xlo, xhi, ylo, yhi as order keys
     std::vector<int64_t> chunk_start;  // [n_exp+1] first chunk of exposure e
     std::vector<int32_t> chunk_box;    // [n_chunks][4], coordinates relative to (x0, y0)
+    std::vector<float> chunk_top;      // [n_chunks] largest ierr
     std::vector<float> x0, y0;         // [n_exp] pixel origin of each exposure
     DevVec<float> data, ierr, xpix, ypix, residual;
     DevVec<float> rad2, D, crpix, crval, CW;
@@ -337,6 +344,7 @@ struct HostPlan {
     std::vector<SrcDesc> srcs;
     std::vector<PatchOut> pouts;
     int64_t n_gauss = 0, n_part = 0, n_pairs = 0, npix = 0;
+    int64_t n_flags = 0;  // flag words of the two-launch pixel pass
     int32_t max_ng = 0;   // most image Gaussians of one exposure
 };
 
@@ -408,6 +416,11 @@ void plan_patch(const fpho_patch *p, int K, int64_t src_base, int64_t chi2_base,
                     t.ylo = std::min(t.ylo, p->chunk_box[4 * c + 2]);
                     t.yhi = std::max(t.yhi, p->chunk_box[4 * c + 3]);
                 }
+                float top = 0.0f;
+                for (int64_t c = c0; c < c1; ++c) top = std::max(top, p->chunk_top[c]);
+                t.tmin = top > 0.0f ? kBrightSigma / top : HUGE_VALF;
+                t.flag = (int32_t)std::min<int64_t>(hp.n_flags, INT32_MAX);
+                hp.n_flags += (int64_t)K * ((ns * np + kWave - 1) / kWave);
                 hp.n_part += (int64_t)ns * kNParams;
                 hp.tiles.push_back(t);
                 // cost model: both passes visit every (pixel, Gaussian) pair
@@ -446,6 +459,41 @@ std::vector<int32_t> cost_order(const HostPlan &hp) {
     return queue;
 }
 
+// Whether a plan's pixel pass goes in two launches (residual_kernel,
+// gradient_kernel) instead of one wave per tile.  One wave per tile needs
+// several tiles per wave slot before the waves end together: with 8 or fewer
+// the two launches are faster for every shape measured (us, one wave per
+// tile / two launches: 357 tiles 1012 / 189, 2659 1140 / 420, 13460 1448 /
+// 1041, 26432 2152 / 1955, 52699 2280 / 2174), above it they lose the work
+// that a tile's slots share (106394 tiles 7329 / 7678, 211725 8080 / 8385).
+// A plan with more than 2^26 flag words (512 MiB: thousands of Gaussians on
+// every pixel) takes one wave per tile too, so the workspace stays bounded.
+bool two_launches(const HostPlan &hp) {
+    const int64_t wave_slots = (int64_t)32 * cu_count_cached();
+    return (int64_t)hp.tiles.size() <= 8 * wave_slots && hp.n_flags <= (int64_t)1 << 26;
+}
+
+// The wave list and buffers of the two-launch pixel pass.
+int build_two_launches(const HostPlan &hp, const std::vector<int32_t> &queue, Plan &plan) {
+    std::vector<int32_t> start(queue.size());
+    int64_t n_items = 0;
+    for (size_t q = 0; q < queue.size(); ++q) {
+        start[q] = (int32_t)n_items;
+        n_items += hp.exps[hp.tiles[queue[q]].exp].n_src + 1;
+    }
+    DevVec<int32_t> start_dev;
+    HIP_TRY(start_dev.upload(start.data(), (int64_t)start.size()));
+    HIP_TRY(plan.items.alloc(n_items));
+    HIP_TRY(launch_list_items(plan.tiles.ptr, plan.queue.ptr, plan.exps.ptr, start_dev.ptr,
+                              (int64_t)queue.size(), plan.items.ptr, nullptr));
+    HIP_TRY(plan.hot.alloc(hp.n_gauss));
+    HIP_TRY(plan.flags.alloc(hp.n_flags));
+    HIP_TRY(plan.resid.alloc((int64_t)hp.slot_boxes.size() * kWave));
+    HIP_TRY(plan.weight.alloc((int64_t)hp.slot_boxes.size() * kWave));
+    HIP_TRY(hipStreamSynchronize(nullptr));   // start_dev goes, other streams read the list
+    return FPHO_OK;
+}
+
 // On failure the plan stays invalid (its buffers may be partly replaced).
 int build_plan(const std::vector<fpho_patch *> &patches, const fpho_launch &launch,
                Plan &plan) {
@@ -482,6 +530,15 @@ int build_plan(const std::vector<fpho_patch *> &patches, const fpho_launch &laun
     HIP_TRY(plan.gauss.alloc(hp.n_gauss));
     HIP_TRY(plan.gauss64.alloc(hp.n_gauss));
     HIP_TRY(plan.gboxes.alloc(hp.n_gauss));
+    plan.hot.release();
+    plan.items.release();
+    plan.flags.release();
+    plan.resid.release();
+    plan.weight.release();
+    if (two_launches(hp)) {
+        const int rc = build_two_launches(hp, queue, plan);
+        if (rc) return rc;
+    }
     HIP_TRY(plan.gpart.alloc(std::max<int64_t>(hp.n_part, 1)));
     HIP_TRY(plan.cpart.alloc(std::max<int64_t>((int64_t)hp.tiles.size(), 1)));
     HIP_TRY(plan.counter.alloc(1));
@@ -521,6 +578,13 @@ struct PlanPtrs {
     ImgGauss *gauss = nullptr;
     ImgGauss64 *gauss64 = nullptr;
     int4 *gboxes = nullptr;
+    // two-launch pixel pass (n_items = 0: one wave per tile)
+    HotGauss *hot = nullptr;
+    const int2 *items = nullptr;
+    uint64_t *flags = nullptr;
+    double *resid = nullptr;
+    float *weight = nullptr;
+    int64_t n_items = 0;
     float *gpart = nullptr;
     double *cpart = nullptr;
     int32_t *counter = nullptr;
@@ -543,6 +607,12 @@ PlanPtrs plan_ptrs(Plan &plan, uint32_t *status) {
     q.gauss = plan.gauss.ptr;
     q.gauss64 = plan.gauss64.ptr;
     q.gboxes = plan.gboxes.ptr;
+    q.hot = plan.hot.ptr;
+    q.items = plan.items.ptr;
+    q.flags = plan.flags.ptr;
+    q.resid = plan.resid.ptr;
+    q.weight = plan.weight.ptr;
+    q.n_items = plan.items.n;
     q.gpart = plan.gpart.ptr;
     q.cpart = plan.cpart.ptr;
     q.counter = plan.counter.ptr;
@@ -582,6 +652,12 @@ EvalArgs eval_args(const PlanPtrs &q) {
     a.grid = std::min<int64_t>(groups_needed,
                                (int64_t)q.launch.groups_per_cu * cu_count_cached());
     if (a.grid < 1) a.grid = 1;
+    a.hot = q.hot;
+    a.items = q.items;
+    a.n_items = q.n_items;
+    a.flags = q.flags;
+    a.resid = q.resid;
+    a.weight = q.weight;
     return a;
 }
 
@@ -592,7 +668,7 @@ template <typename Src>
 int run_ptrs(const PlanPtrs &q, const Src *props, double *chi2, double *dchi2,
              hipStream_t stream) {
     if (q.timing) HIP_TRY(hipEventRecord(q.ev[0], stream));
-    HIP_TRY(launch_convert(q.exps, q.n_exp, props, q.gauss, q.gauss64, q.gboxes, q.status,
+    HIP_TRY(launch_convert(q.exps, q.n_exp, props, q.gauss, q.gauss64, q.gboxes, q.hot, q.status,
                            stream));
     const EvalArgs a = eval_args(q);
     if (q.timing) HIP_TRY(hipEventRecord(q.ev[1], stream));
@@ -811,6 +887,10 @@ int fpho_patch_create(const fpho_patch_desc *d, int return_residual, fpho_patch 
                 ylo = std::min(ylo, d->ypix[i] - oy);
                 yhi = std::max(yhi, d->ypix[i] - oy);
             }
+            float top = 0.0f;
+            for (int64_t i = s0 + c; i < s0 + std::min<int64_t>(n, c + kWave); ++i)
+                top = std::max(top, d->ierr[i]);
+            p->chunk_top.push_back(top);
             p->chunk_box.push_back(order_key(xlo));
             p->chunk_box.push_back(order_key(xhi));
             p->chunk_box.push_back(order_key(ylo));
@@ -1008,6 +1088,8 @@ int fpho_evaluate_async_noalloc(fpho_patch *p, const fpho_source *prop_dev, doub
     q.cpart = reinterpret_cast<double *>(base + o_cpart);
     q.counter = reinterpret_cast<int32_t *>(base + o_counter);
     q.timing = false;
+    q.hot = nullptr;   // one wave per tile: its work buffers fit the scratch array
+    q.n_items = 0;
     return run_ptrs(q, prop_dev, chi2_dev, dchi2_dev, (hipStream_t)stream);
 }
 

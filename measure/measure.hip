@@ -294,7 +294,8 @@ int fpho_measure_batch_count_pairs(fpho_batch *b, const fpho_source *props, int6
     if (err == hipSuccess)
         err = launch_convert(v.eval.exps, v.n_exp, props, const_cast<ImgGauss *>(v.eval.gauss),
                              const_cast<ImgGauss64 *>(v.eval.gauss64),
-                             const_cast<int4 *>(v.eval.gboxes), v.status, nullptr);
+                             const_cast<int4 *>(v.eval.gboxes),
+                             const_cast<HotGauss *>(v.eval.hot), v.status, nullptr);
     if (err == hipSuccess && v.eval.n_tiles > 0) {
         const int W = v.eval.waves_per_group;
         const unsigned groups = (unsigned)((v.eval.n_tiles + W - 1) / W);
