@@ -51,10 +51,12 @@ struct SplineView {
     double nsersic_min;
 };
 
-hipError_t launch_convert(const ExpDesc *exps, int64_t n_exp, const fpho_source *props,
+hipError_t launch_convert(const ExpDesc *exps, int64_t n_exp, int32_t max_ng,
+                          const fpho_source *props,
                           ImgGauss *out, ImgGauss64 *out64, int4 *boxes, HotGauss *hot,
                           uint32_t *status, hipStream_t stream);
-hipError_t launch_convert(const ExpDesc *exps, int64_t n_exp, const Source64 *props,
+hipError_t launch_convert(const ExpDesc *exps, int64_t n_exp, int32_t max_ng,
+                          const Source64 *props,
                           ImgGauss *out, ImgGauss64 *out64, int4 *boxes, HotGauss *hot,
                           uint32_t *status, hipStream_t stream);
 hipError_t launch_eval(const EvalArgs &a, hipStream_t stream);
@@ -79,6 +81,7 @@ hipError_t launch_stack(const SrcDesc *srcs, int64_t n_srcs, const PatchOut *pou
 struct PlanView {
     EvalArgs eval;
     int64_t n_exp;
+    int32_t max_ng;
     uint32_t *status;
 };
 int batch_plan_view(fpho_batch *b, PlanView *out);

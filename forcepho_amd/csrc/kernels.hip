@@ -21,6 +21,8 @@
 //                       (forcepho/model.py:331-332,370-387)
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "fpho_internal.h"
 #include "kernels.h"
 
@@ -162,16 +164,22 @@ __device__ __forceinline__ uint32_t make_image_gaussian(const ExpDesc &e, const 
     return flags;
 }
 
-// One workgroup per exposure; lanes stride over its n_src * n_psf Gaussians.
+// Workgroups (exposure, part): one wave each, its lanes stride over the
+// exposure's n_src * n_psf Gaussians in steps of gridDim.y waves.  Bound by the
+// latency of one Gaussian's FP64 chain (sincos, divisions, square roots), so
+// the Gaussians are spread until the chip holds a wave or two per SIMD; one
+// workgroup of 128 lanes per exposure ran a chain per 128 Gaussians (us, before
+// -> after: four patches of up to 1620 Gaussians an exposure 20.7 -> 9.8, 24
+// exposures of 2160 46.6 -> 9.4, 96 patches 116 -> 106).
 // Invalid inputs set bits of *status (a vector atomic, taken only then).
 template <typename Src>
-__global__ __launch_bounds__(128) void convert_kernel(
+__global__ __launch_bounds__(kWave) void convert_kernel(
     const ExpDesc *__restrict__ exps, const Src *__restrict__ props,
     ImgGauss *__restrict__ out, ImgGauss64 *__restrict__ out64, int4 *__restrict__ boxes,
     HotGauss *__restrict__ hot, uint32_t *__restrict__ status) {
-    const ExpDesc e = exps[blockIdx.x];
+    const ExpDesc &e = exps[blockIdx.x];
     const int n = e.n_src * e.n_psf;
-    for (int j = threadIdx.x; j < n; j += blockDim.x) {
+    for (int j = blockIdx.y * kWave + threadIdx.x; j < n; j += gridDim.y * kWave) {
         const int s = j / e.n_psf;
         const int p = j - s * e.n_psf;
         ImgGauss g;
@@ -1106,38 +1114,25 @@ __device__ inline int knot_span(const double *t, int n_t, double x) {
     return lo;
 }
 
-// Writes the FP32 record to props and/or the FP64 record to props64 (either
-// may be null).
-__global__ __launch_bounds__(64) void theta_kernel(
-    const SrcDesc *__restrict__ srcs, int32_t n_srcs, const double *__restrict__ theta,
-    SplineView sp, fpho_source *__restrict__ props, Source64 *__restrict__ props64,
+// One wave per source: lane m evaluates mixture component m, and the wave
+// writes the FP32 record to props and/or the FP64 record to props64 (either
+// may be null).  Bound by the latency of the knot search and of a component's
+// 16 coefficients; one lane per source ran the components one after another
+// (us, before -> after: four patches 10.7 -> 4.7, 96 patches 21.5 -> 7.2).
+__global__ __launch_bounds__(kWave) void theta_kernel(
+    const SrcDesc *__restrict__ srcs, const double *__restrict__ theta, SplineView sp,
+    fpho_source *__restrict__ props, Source64 *__restrict__ props64,
     uint32_t *__restrict__ status) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n_srcs) return;
-    const SrcDesc sd = srcs[i];
+    const int lane = threadIdx.x;
+    const SrcDesc sd = srcs[blockIdx.x];
     const double *th = theta + sd.theta_off;
-    {
-        bool finite = true;
-        for (int j = 0; j < sd.n_bands + 6; ++j) finite = finite && isfinite(th[j]);
-        if (!finite) atomicOr(status, FPHO_STATUS_THETA_NONFINITE);
-    }
-    Source64 o;
-    for (int b = 0; b < FPHO_MAXBANDS; ++b) o.fluxes[b] = 0.0;
-    for (int m = 0; m < FPHO_MAXRADII; ++m) {
-        o.mixture_amplitudes[m] = 0.0;
-        o.damplitude_drh[m] = 0.0;
-        o.damplitude_dnsersic[m] = 0.0;
-    }
     const int nb = sd.n_bands;
-    for (int b = 0; b < nb; ++b) o.fluxes[b] = th[b];
-    o.ra = th[nb + 0];
-    o.dec = th[nb + 1];
-    o.q = th[nb + 2];
-    o.pa = th[nb + 3];
-    o.nsersic = th[nb + 4];
-    o.rh = th[nb + 5];
-    const double n = o.nsersic, rh = o.rh;
+    const double v = lane < nb + 6 ? th[lane] : 0.0;   // nb + 6 <= 36
+    if (__builtin_amdgcn_ballot_w64(!isfinite(v)) != 0 && lane == 0)
+        atomicOr(status, FPHO_STATUS_THETA_NONFINITE);
+    const double n = th[nb + 4], rh = th[nb + 5];
 
+    double amp = 0.0, amp_n = 0.0, amp_r = 0.0;   // component `lane`
     if (n < sp.nsersic_min) {
         // one-hot at the radius closest to rh (forcepho/sources.py:662-665)
         int best = 0;
@@ -1149,9 +1144,9 @@ __global__ __launch_bounds__(64) void theta_kernel(
                 best = m;
             }
         }
-        o.mixture_amplitudes[best] = 1.0;
+        amp = lane == best ? 1.0 : 0.0;
     } else if (rh < 0.0) {
-        o.mixture_amplitudes[0] = 1.0;  // forcepho/sources.py:666-668
+        amp = lane == 0 ? 1.0 : 0.0;  // forcepho/sources.py:666-668
     } else {
         const double xn = fmin(fmax(n, sp.tx[3]), sp.tx[sp.n_tx - 4]);
         const double xr = fmin(fmax(rh, sp.ty[3]), sp.ty[sp.n_ty - 4]);
@@ -1162,66 +1157,79 @@ __global__ __launch_bounds__(64) void theta_kernel(
         bspline3(sp.ty, ly, xr, Ny, dNy);
         const int ny = sp.n_ty - 4;
         const int nx = sp.n_tx - 4;
-        for (int m = 0; m < sp.n_amp; ++m) {
-            const double *c = sp.coeffs + (int64_t)m * nx * ny;
-            double v = 0.0, vn = 0.0, vr = 0.0;
+        if (lane < sp.n_amp) {
+            const double *c = sp.coeffs + (int64_t)lane * nx * ny;
+#pragma unroll
             for (int a = 0; a < 4; ++a) {
                 const double *row = c + (int64_t)(lx - 3 + a) * ny + (ly - 3);
                 double rv = 0.0, rd = 0.0;
+#pragma unroll
                 for (int b = 0; b < 4; ++b) {
                     rv += row[b] * Ny[b];
                     rd += row[b] * dNy[b];
                 }
-                v += Nx[a] * rv;
-                vn += dNx[a] * rv;
-                vr += Nx[a] * rd;
+                amp += Nx[a] * rv;
+                amp_n += dNx[a] * rv;
+                amp_r += Nx[a] * rd;
             }
-            o.mixture_amplitudes[m] = v;
-            o.damplitude_dnsersic[m] = vn;
-            o.damplitude_drh[m] = vr;
         }
     }
-    if (props64) props64[sd.proposal] = o;
-    if (props) {
-        fpho_source f;
-        f.ra = (float)o.ra;
-        f.dec = (float)o.dec;
-        f.q = (float)o.q;
-        f.pa = (float)o.pa;
-        f.nsersic = (float)o.nsersic;
-        f.rh = (float)o.rh;
-        for (int b = 0; b < FPHO_MAXBANDS; ++b) f.fluxes[b] = (float)o.fluxes[b];
-        for (int m = 0; m < FPHO_MAXRADII; ++m) {
-            f.mixture_amplitudes[m] = (float)o.mixture_amplitudes[m];
-            f.damplitude_drh[m] = (float)o.damplitude_drh[m];
-            f.damplitude_dnsersic[m] = (float)o.damplitude_dnsersic[m];
+    // fields in record order: ra, dec, q, pa, nsersic, rh, then the arrays
+    const double shape = lane < 6 ? th[nb + lane] : 0.0;
+    const double flux = lane < nb ? v : 0.0;
+    if (props64) {
+        Source64 &o = props64[sd.proposal];
+        if (lane < 6) (&o.ra)[lane] = shape;
+        if (lane < FPHO_MAXBANDS) o.fluxes[lane] = flux;
+        if (lane < FPHO_MAXRADII) {
+            o.mixture_amplitudes[lane] = amp;
+            o.damplitude_drh[lane] = amp_r;
+            o.damplitude_dnsersic[lane] = amp_n;
         }
-        props[sd.proposal] = f;
+    }
+    if (props) {
+        fpho_source &f = props[sd.proposal];
+        if (lane < 6) (&f.ra)[lane] = (float)shape;
+        if (lane < FPHO_MAXBANDS) f.fluxes[lane] = (float)flux;
+        if (lane < FPHO_MAXRADII) {
+            f.mixture_amplitudes[lane] = (float)amp;
+            f.damplitude_drh[lane] = (float)amp_r;
+            f.damplitude_dnsersic[lane] = (float)amp_n;
+        }
     }
 }
 
 // ------------------------------------------------------- gradient stacking
 
-__global__ __launch_bounds__(64) void stack_kernel(
+// One wave per source (lane: parameter of its block), then one lane per patch.
+// Latency bound: a lane's loads over the bands are independent, the bands are
+// added in order (us, one lane per source -> one wave: four patches 5.9 ->
+// 4.6, 96 patches 12.6 -> 4.8).
+__global__ __launch_bounds__(kWave) void stack_kernel(
     const SrcDesc *__restrict__ srcs, int32_t n_srcs, const PatchOut *__restrict__ pouts,
     int32_t n_patches, const double *__restrict__ chi2, const double *__restrict__ dchi2,
     double *__restrict__ lnlike, double *__restrict__ grad) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n_srcs) {
-        const SrcDesc sd = srcs[i];
+    const int lane = threadIdx.x;
+    if ((int)blockIdx.x < n_srcs) {
+        const SrcDesc sd = srcs[blockIdx.x];
         const double *dv = dchi2 + sd.dchi2_base;
-        double *gv = grad + sd.theta_off;
         const int nb = sd.n_bands;
-        for (int b = 0; b < nb; ++b) gv[b] = -0.5 * dv[(int64_t)b * sd.src_stride];
-        for (int j = 1; j < kNParams; ++j) {
+        if (lane < nb) {
+            grad[sd.theta_off + lane] = -0.5 * dv[(int64_t)lane * sd.src_stride];
+        } else if (lane < nb + kNParams - 1) {
+            const double *col = dv + lane - nb + 1;
             double acc = 0.0;
-            for (int b = 0; b < nb; ++b) acc += dv[(int64_t)b * sd.src_stride + j];
-            gv[nb + j - 1] = -0.5 * acc;
+#pragma unroll 4
+            for (int b = 0; b < nb; ++b) acc += col[(int64_t)b * sd.src_stride];
+            grad[sd.theta_off + lane] = -0.5 * acc;
         }
+        return;
     }
+    const int i = ((int)blockIdx.x - n_srcs) * kWave + lane;
     if (i < n_patches) {
         const PatchOut po = pouts[i];
         double acc = 0.0;
+#pragma unroll 4
         for (int b = 0; b < po.n_bands; ++b) acc += chi2[po.chi2_off + b];
         lnlike[i] = -0.5 * acc;
     }
@@ -1244,25 +1252,30 @@ __global__ __launch_bounds__(256) void response_kernel(const double *__restrict_
 // ---------------------------------------------------------------- launchers
 
 template <typename Src>
-static hipError_t launch_convert_t(const ExpDesc *exps, int64_t n_exp, const Src *props,
+static hipError_t launch_convert_t(const ExpDesc *exps, int64_t n_exp, int32_t max_ng, const Src *props,
                                    ImgGauss *out, ImgGauss64 *out64, int4 *boxes, HotGauss *hot,
                                    uint32_t *status, hipStream_t stream) {
     if (n_exp <= 0) return hipSuccess;
-    hipLaunchKernelGGL(convert_kernel<Src>, dim3((unsigned)n_exp), dim3(128), 0, stream,
-                       exps, props, out, out64, boxes, hot, status);
+    // a wave per 64 Gaussians until there are 16384 waves (64 per CU)
+    const int64_t blocks = std::max(1, (max_ng + kWave - 1) / kWave);
+    const int64_t parts = std::min(blocks, std::max<int64_t>(1, 16384 / n_exp));
+    hipLaunchKernelGGL(convert_kernel<Src>, dim3((unsigned)n_exp, (unsigned)parts), dim3(kWave),
+                       0, stream, exps, props, out, out64, boxes, hot, status);
     return hipGetLastError();
 }
 
-hipError_t launch_convert(const ExpDesc *exps, int64_t n_exp, const fpho_source *props,
+hipError_t launch_convert(const ExpDesc *exps, int64_t n_exp, int32_t max_ng,
+                          const fpho_source *props,
                           ImgGauss *out, ImgGauss64 *out64, int4 *boxes, HotGauss *hot,
                           uint32_t *status, hipStream_t stream) {
-    return launch_convert_t(exps, n_exp, props, out, out64, boxes, hot, status, stream);
+    return launch_convert_t(exps, n_exp, max_ng, props, out, out64, boxes, hot, status, stream);
 }
 
-hipError_t launch_convert(const ExpDesc *exps, int64_t n_exp, const Source64 *props,
+hipError_t launch_convert(const ExpDesc *exps, int64_t n_exp, int32_t max_ng,
+                          const Source64 *props,
                           ImgGauss *out, ImgGauss64 *out64, int4 *boxes, HotGauss *hot,
                           uint32_t *status, hipStream_t stream) {
-    return launch_convert_t(exps, n_exp, props, out, out64, boxes, hot, status, stream);
+    return launch_convert_t(exps, n_exp, max_ng, props, out, out64, boxes, hot, status, stream);
 }
 
 hipError_t launch_response(const double *dchi2, int32_t n_bands, int32_t n_src,
@@ -1349,19 +1362,17 @@ hipError_t launch_theta(const SrcDesc *srcs, int64_t n_srcs, const double *theta
                         const SplineView &sp, fpho_source *props, Source64 *props64,
                         uint32_t *status, hipStream_t stream) {
     if (n_srcs <= 0) return hipSuccess;
-    const unsigned blocks = (unsigned)((n_srcs + 63) / 64);
-    hipLaunchKernelGGL(theta_kernel, dim3(blocks), dim3(64), 0, stream, srcs, (int32_t)n_srcs,
-                       theta, sp, props, props64, status);
+    hipLaunchKernelGGL(theta_kernel, dim3((unsigned)n_srcs), dim3(kWave), 0, stream, srcs, theta,
+                       sp, props, props64, status);
     return hipGetLastError();
 }
 
 hipError_t launch_stack(const SrcDesc *srcs, int64_t n_srcs, const PatchOut *pouts,
                         int64_t n_patches, const double *chi2, const double *dchi2,
                         double *lnlike, double *grad, hipStream_t stream) {
-    const int64_t n = n_srcs > n_patches ? n_srcs : n_patches;
+    const int64_t n = n_srcs + (n_patches + kWave - 1) / kWave;
     if (n <= 0) return hipSuccess;
-    const unsigned blocks = (unsigned)((n + 63) / 64);
-    hipLaunchKernelGGL(stack_kernel, dim3(blocks), dim3(64), 0, stream, srcs, (int32_t)n_srcs,
+    hipLaunchKernelGGL(stack_kernel, dim3((unsigned)n), dim3(kWave), 0, stream, srcs, (int32_t)n_srcs,
                        pouts, (int32_t)n_patches, chi2, dchi2, lnlike, grad);
     return hipGetLastError();
 }

@@ -668,8 +668,8 @@ template <typename Src>
 int run_ptrs(const PlanPtrs &q, const Src *props, double *chi2, double *dchi2,
              hipStream_t stream) {
     if (q.timing) HIP_TRY(hipEventRecord(q.ev[0], stream));
-    HIP_TRY(launch_convert(q.exps, q.n_exp, props, q.gauss, q.gauss64, q.gboxes, q.hot, q.status,
-                           stream));
+    HIP_TRY(launch_convert(q.exps, q.n_exp, q.max_ng, props, q.gauss, q.gauss64, q.gboxes, q.hot,
+                           q.status, stream));
     const EvalArgs a = eval_args(q);
     if (q.timing) HIP_TRY(hipEventRecord(q.ev[1], stream));
     HIP_TRY(launch_eval(a, stream));
@@ -1316,6 +1316,7 @@ int batch_plan_view(fpho_batch *b, PlanView *out) {
     if (rc) return rc;
     out->eval = eval_args(b->plan);
     out->n_exp = b->plan.n_exp;
+    out->max_ng = b->plan.max_ng;
     out->status = b->plan.status.ptr;
     return FPHO_OK;
 }

@@ -292,7 +292,8 @@ int fpho_measure_batch_count_pairs(fpho_batch *b, const fpho_source *props, int6
     if (err != hipSuccess) return fail("hipMalloc", err);
     err = hipMemset(cnt, 0, sizeof(unsigned long long));
     if (err == hipSuccess)
-        err = launch_convert(v.eval.exps, v.n_exp, props, const_cast<ImgGauss *>(v.eval.gauss),
+        err = launch_convert(v.eval.exps, v.n_exp, v.max_ng, props,
+                             const_cast<ImgGauss *>(v.eval.gauss),
                              const_cast<ImgGauss64 *>(v.eval.gauss64),
                              const_cast<int4 *>(v.eval.gboxes),
                              const_cast<HotGauss *>(v.eval.hot), v.status, nullptr);
