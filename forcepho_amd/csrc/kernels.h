@@ -65,7 +65,8 @@ hipError_t launch_list_items(const TileDesc *tiles, const int32_t *queue, const 
                              hipStream_t stream);
 hipError_t launch_response(const double *dchi2, int32_t n_bands, int32_t n_src,
                            fpho_response *out, hipStream_t stream);
-hipError_t launch_reduce(const OutDesc *outs, int64_t n_outs, const float *gpart,
+// max_src: most sources of one patch
+hipError_t launch_reduce(const OutDesc *outs, int64_t n_outs, int32_t max_src, const float *gpart,
                          const double *cpart, double *chi2, double *dchi2, int fp64,
                          hipStream_t stream);
 hipError_t launch_theta(const SrcDesc *srcs, int64_t n_srcs, const double *theta,

@@ -1012,55 +1012,63 @@ __global__ void zero_counter_kernel(int32_t *counter) {
 
 // ------------------------------------------------------------------ reduce
 
-// One workgroup per (patch, band).  Column j of the band's [ntiles][n_src*7]
+// Workgroups (patch-band, 64 columns).  Column j of the band's [ntiles][n_src*7]
 // partial block is cut into S segments of consecutive tiles, S a function of
 // the column count only (S * ncol <= kReduceSlots); each segment is summed in
 // tile order by one lane, then each column's S segment sums in segment
-// order.  chi2 partials go through a fixed-shape tree.  The result depends
-// only on (ntiles, ncol), not on tile execution order or the launch.
+// order.  chi2 partials go through a fixed-shape tree (first column group).
+// The result depends only on (ntiles, ncol), not on tile execution order or
+// the launch.  Bound by load latency: a single patch has few (patch, band)
+// groups, so the columns are spread over workgroups and a lane keeps 16 loads
+// in flight (us, one workgroup and 4 loads -> these: 12 bands x 512 tiles x
+// 420 columns 24.0 -> 6.2; 10 x 2304 x 91 28.6 -> 12.7; 96 patches 41 -> 26).
 constexpr int kReduceSlots = 4096;
-constexpr int kReduceThreads = 1024;   // a single patch has few (patch, band) groups
+constexpr int kReduceCols = 64;        // columns per workgroup
+constexpr int kReduceSegs = 16;        // S at most
+constexpr int kReduceThreads = kReduceCols * kReduceSegs;
 
 template <typename Acc>
 __global__ __launch_bounds__(kReduceThreads) void reduce_kernel(
     const OutDesc *__restrict__ outs, const float *__restrict__ gpart,
     const double *__restrict__ cpart, double *__restrict__ chi2,
     double *__restrict__ dchi2) {
-    __shared__ Acc seg[kReduceSlots];
+    __shared__ Acc seg[kReduceThreads];
     __shared__ Acc sh[kReduceThreads];
     const OutDesc o = outs[blockIdx.x];
     const int ncol = o.n_src * kNParams;
-    const int S = max(1, min(16, kReduceSlots / ncol));
+    const int j0 = blockIdx.y * kReduceCols;
+    if (j0 >= ncol) return;
+    const int S = max(1, min(kReduceSegs, kReduceSlots / ncol));
     const int len = (o.ntiles + S - 1) / S;   // tiles per segment
-    for (int w = threadIdx.x; w < ncol * S; w += blockDim.x) {
-        const int j = w % ncol, r = w / ncol;
+    const int j = j0 + threadIdx.x % kReduceCols, r = threadIdx.x / kReduceCols;
+    if (j < ncol && r < S) {
         const int t0 = r * len, t1 = min(o.ntiles, t0 + len);
         const float *col = gpart + o.part0 + j;
         Acc acc = 0;
         int t = t0;
-        for (; t + 4 <= t1; t += 4) {
-            const float v0 = col[(int64_t)(t + 0) * ncol];
-            const float v1 = col[(int64_t)(t + 1) * ncol];
-            const float v2 = col[(int64_t)(t + 2) * ncol];
-            const float v3 = col[(int64_t)(t + 3) * ncol];
-            acc += (Acc)v0;
-            acc += (Acc)v1;
-            acc += (Acc)v2;
-            acc += (Acc)v3;
+        for (; t + 16 <= t1; t += 16) {
+            float v[16];
+#pragma unroll
+            for (int u = 0; u < 16; ++u) v[u] = col[(int64_t)(t + u) * ncol];
+#pragma unroll
+            for (int u = 0; u < 16; ++u) acc += (Acc)v[u];
         }
+#pragma unroll 4
         for (; t < t1; ++t) acc += (Acc)col[(int64_t)t * ncol];
-        seg[r * ncol + j] = acc;
+        seg[threadIdx.x] = acc;
     }
     Acc c = 0;
-    for (int t = threadIdx.x; t < o.ntiles; t += blockDim.x) c += (Acc)cpart[o.tile0 + t];
+    if (j0 == 0)
+        for (int t = threadIdx.x; t < o.ntiles; t += kReduceThreads) c += (Acc)cpart[o.tile0 + t];
     sh[threadIdx.x] = c;
     __syncthreads();
-    for (int j = threadIdx.x; j < ncol; j += blockDim.x) {
+    if (r == 0 && j < ncol) {
         Acc acc = 0;
-        for (int r = 0; r < S; ++r) acc += seg[r * ncol + j];
+        for (int q = 0; q < S; ++q) acc += seg[q * kReduceCols + threadIdx.x];
         dchi2[o.dchi2_out + j] = (double)acc;
     }
-    for (int w = blockDim.x / 2; w > 0; w >>= 1) {
+    if (j0 > 0) return;
+    for (int w = kReduceThreads / 2; w > 0; w >>= 1) {
         if ((int)threadIdx.x < w) sh[threadIdx.x] += sh[threadIdx.x + w];
         __syncthreads();
     }
@@ -1345,16 +1353,18 @@ hipError_t launch_list_items(const TileDesc *tiles, const int32_t *queue, const 
     return hipGetLastError();
 }
 
-hipError_t launch_reduce(const OutDesc *outs, int64_t n_outs, const float *gpart,
+hipError_t launch_reduce(const OutDesc *outs, int64_t n_outs, int32_t max_src, const float *gpart,
                          const double *cpart, double *chi2, double *dchi2, int fp64,
                          hipStream_t stream) {
     if (n_outs <= 0) return hipSuccess;
+    const dim3 grid((unsigned)n_outs,
+                    (unsigned)((max_src * kNParams + kReduceCols - 1) / kReduceCols));
     if (fp64)
-        hipLaunchKernelGGL(reduce_kernel<double>, dim3((unsigned)n_outs), dim3(kReduceThreads), 0,
-                           stream, outs, gpart, cpart, chi2, dchi2);
+        hipLaunchKernelGGL(reduce_kernel<double>, grid, dim3(kReduceThreads), 0, stream, outs,
+                           gpart, cpart, chi2, dchi2);
     else
-        hipLaunchKernelGGL(reduce_kernel<float>, dim3((unsigned)n_outs), dim3(kReduceThreads), 0,
-                           stream, outs, gpart, cpart, chi2, dchi2);
+        hipLaunchKernelGGL(reduce_kernel<float>, grid, dim3(kReduceThreads), 0, stream, outs,
+                           gpart, cpart, chi2, dchi2);
     return hipGetLastError();
 }
 

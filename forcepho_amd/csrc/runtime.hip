@@ -177,6 +177,7 @@ struct Plan {
     int64_t n_exp = 0, n_tiles = 0, n_outs = 0, n_gauss = 0, n_srcs = 0, n_patches = 0;
     int64_t n_pairs = 0, npix = 0, n_part = 0;
     int32_t max_ng = 0;  // most image Gaussians of one exposure
+    int32_t max_src = 0; // most sources of one patch
     std::vector<int64_t> src_off, chi2_off, dchi2_off, theta_off;  // per patch, +1
     fpho_launch launch;
     int precision = kPrecMixed;
@@ -558,6 +559,8 @@ int build_plan(const std::vector<fpho_patch *> &patches, const fpho_launch &laun
     plan.n_gauss = hp.n_gauss;
     plan.n_part = hp.n_part;
     plan.max_ng = hp.max_ng;
+    plan.max_src = 0;
+    for (const fpho_patch *p : patches) plan.max_src = std::max(plan.max_src, p->n_sources);
     plan.n_srcs = (int64_t)hp.srcs.size();
     plan.n_patches = (int64_t)patches.size();
     plan.n_pairs = hp.n_pairs;
@@ -590,7 +593,7 @@ struct PlanPtrs {
     int32_t *counter = nullptr;
     uint32_t *status = nullptr;
     int64_t n_exp = 0, n_tiles = 0, n_outs = 0;
-    int32_t max_ng = 0;
+    int32_t max_ng = 0, max_src = 0;
     fpho_launch launch;
     int precision = kPrecMixed;
     bool timing = false;
@@ -621,6 +624,7 @@ PlanPtrs plan_ptrs(Plan &plan, uint32_t *status) {
     q.n_tiles = plan.n_tiles;
     q.n_outs = plan.n_outs;
     q.max_ng = plan.max_ng;
+    q.max_src = plan.max_src;
     q.launch = plan.launch;
     q.precision = plan.precision;
     q.timing = plan.timing;
@@ -674,7 +678,7 @@ int run_ptrs(const PlanPtrs &q, const Src *props, double *chi2, double *dchi2,
     if (q.timing) HIP_TRY(hipEventRecord(q.ev[1], stream));
     HIP_TRY(launch_eval(a, stream));
     if (q.timing) HIP_TRY(hipEventRecord(q.ev[2], stream));
-    HIP_TRY(launch_reduce(q.outs, q.n_outs, q.gpart, q.cpart, chi2, dchi2,
+    HIP_TRY(launch_reduce(q.outs, q.n_outs, q.max_src, q.gpart, q.cpart, chi2, dchi2,
                           q.precision != kPrecFP32, stream));
     if (q.timing) HIP_TRY(hipEventRecord(q.ev[3], stream));
     return FPHO_OK;
