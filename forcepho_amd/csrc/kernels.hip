@@ -190,7 +190,7 @@ __global__ __launch_bounds__(kWave) void convert_kernel(
         out64[e.gauss_off + j] = g64;
         boxes[e.gauss_off + j] = make_int4(g.xlo, g.xhi, g.ylo, g.yhi);
         if (hot)
-            hot[e.gauss_off + j] = {g.xcen, g.ycen, g.sfxx, g.sfyy, g.sfxy, g.hcs, g.ampA, 0.0f};
+            hot[e.gauss_off + j] = {g.xcen, g.ycen, g.sfxx, g.sfyy, g.sfxy, g.hcs, g.ampA, 0};
     }
 }
 
@@ -691,8 +691,21 @@ __global__ __launch_bounds__(256) FPHO_EVAL_OCCUPANCY void eval_persistent_kerne
 //
 // What bounds it: VALU issue, and on small plans the serial chain of the
 // heaviest wave.  Measured (us, one wave per tile -> two launches): 16 tiles
-// of 54 Gaussians 58 -> 33; 2048 tiles of 720 535 -> 311; 6144 tiles of 2160
-// 1440 -> 1206; 575 tiles of up to 1620 (four patches) 882 -> 158.
+// of 54 Gaussians 58 -> 29; 2048 tiles of 720 535 -> 260; 6144 tiles of 2160
+// 1440 -> 980; 575 tiles of up to 1620 (four patches) 882 -> 125.
+
+// xcd_swizzle with the XCDs' chunks moved on by three from row to row: an
+// exposure is often a whole number of chunks, and without that an XCD would
+// take the same part of every exposure, its crowded middle or its empty edge.
+// Chunks of 128 waves once there are several rows of them, else of 64.
+__device__ __forceinline__ int xcd_rotate(int b, int n) {
+    const int shift = n >= 1 << 15 ? 7 : 6;   // log2 of the chunk
+    const int rows = n >> (shift + 3);
+    if (b >= rows << (shift + 3)) return b;
+    const int local = b >> 3, row = local >> shift;
+    const int xcd = (b + 3 * row) & 7;
+    return (((row << 3) + xcd) << shift) + (local & ((1 << shift) - 1));
+}
 
 // A pointer known to be to device memory (descriptors hold generic ones), so
 // loads take a scalar base and a 32-bit lane offset.
@@ -729,19 +742,28 @@ __device__ __forceinline__ int rank_in(uint64_t m) {
                                      __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0));
 }
 
-// Lane values in the order "lanes set in m first" (a permutation of the wave).
-__device__ __forceinline__ uint32_t set_first(uint64_t m, bool set, int lane, uint32_t v) {
-    const int rank = rank_in(m);
-    const int to = set ? rank : __builtin_popcountll(m) + lane - rank;
-    return (uint32_t)__builtin_amdgcn_ds_permute(to << 2, (int)v);
+// LDS written by lanes of this wave is visible to its other lanes.
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// The record of Gaussian i, tagged with i (two 16-byte loads).
+__device__ __forceinline__ HotGauss load_hot(const HotGauss *__restrict__ hot, uint32_t i) {
+    const Global<float4> p = global(reinterpret_cast<const float4 *>(hot)) + 2 * i;
+    const float4 a = *(const float4 *)p, b = *(const float4 *)(p + 1);
+    return {a.x, a.y, a.z, a.w, b.x, b.y, b.z, i};
 }
 
 // Pass 1 of one slot.  Each block of 64 Gaussians is tested at once (lane j:
-// Gaussian base + j) and the ones that meet the slot are listed in a vector
-// register as record offsets, so a visit costs a readlane and a scalar load.
-// kVisits of them go through together: one wait for their records and one
-// test for bright terms (four small patches: 218 us a pass with four at once,
-// 232 with two; eight records do not fit the scalar registers).
+// Gaussian base + j) and the records of those that meet the slot go to LDS in
+// index order, from where a visit reads its own with a broadcast.  A VALU
+// instruction with a scalar operand issues every 4.4 cycles here, one whose
+// operands are all vector registers every 2.6; 8 of a visit's 18 read the
+// record, so taking it from LDS instead of by scalar loads cut the kernel from
+// 460 to 360 us (24576 slots, 2160 Gaussians) and from 142 to 120 (8192, 720).
+// kVisits go through together: one wait for their records and one test for
+// bright terms (four small patches: 218 us a pass with four, 232 with two).
 template <int K, bool MIXED, bool CENTRE>
 __global__ __launch_bounds__(kWave) FPHO_EVAL_OCCUPANCY void residual_kernel(
     const TileDesc *__restrict__ tiles, const int32_t *__restrict__ queue,
@@ -751,7 +773,7 @@ __global__ __launch_bounds__(kWave) FPHO_EVAL_OCCUPANCY void residual_kernel(
     double *__restrict__ resid, float *__restrict__ weight, int32_t cull) {
     constexpr int kVisits = 4;
     const int lane = threadIdx.x;
-    const int wave = xcd_swizzle<kXcdChunk>((int)blockIdx.x, (int)gridDim.x);
+    const int wave = xcd_rotate((int)blockIdx.x, (int)gridDim.x);
     const TileDesc t = tiles[queue[wave / K]];
     const int k = wave % K;
     const int npix = t.npix - k * kWave;   // of this slot and the ones after it
@@ -764,8 +786,6 @@ __global__ __launch_bounds__(kWave) FPHO_EVAL_OCCUPANCY void residual_kernel(
     const float ylo = key_float(box.z) - 0.01f, yhi = key_float(box.w) + 0.01f;
     const ImgGauss *__restrict__ g = gauss + e.gauss_off;
     const ImgGauss64 *__restrict__ g64 = gauss64 + e.gauss_off;
-    const char *__restrict__ gh = reinterpret_cast<const char *>(hot + e.gauss_off);
-    const Global<HotGauss> gv = global(hot + e.gauss_off);
     const int ng = e.n_src * e.n_psf;
 
     float x = kMaskedCoord, y = kMaskedCoord, r = 0.0f, iek = 0.0f;
@@ -778,11 +798,11 @@ __global__ __launch_bounds__(kWave) FPHO_EVAL_OCCUPANCY void residual_kernel(
     double rd = (double)r;
 
     // pass 1 of one visit: the term, and whether a lane is inside the cutoff
-    auto term = [&](const HotGauss &H, float xl, float yl, uint64_t &in_lanes) {
+    auto term = [&](const HotGauss &H, const float2 &L, uint64_t &in_lanes) {
         float dx = x - H.xcen, dy = y - H.ycen, vx, vy;
         if (CENTRE) {   // the pixel offset from the FP64 centre
-            dx -= xl;
-            dy -= yl;
+            dx -= L.x;
+            dy -= L.y;
         }
         const float ea = exponent1(dx, dy, H.sfxx, H.sfyy, H.sfxy, vx, vy);
         const bool in = !(ea < kCutScaled);
@@ -790,7 +810,7 @@ __global__ __launch_bounds__(kWave) FPHO_EVAL_OCCUPANCY void residual_kernel(
         const float gp = cut_exp(in, ea);
         return H.ampA * gp * fmaf(vx, vx, fmaf(vy, vy, H.hcs));
     };
-    auto subtract_bright = [&](float c, uint32_t off) {
+    auto subtract_bright = [&](float c, const HotGauss &H) {
         if (__builtin_amdgcn_ballot_w64(fabsf(c) > t.tmin) == 0) {
             rd -= (double)c;
             return;
@@ -799,30 +819,36 @@ __global__ __launch_bounds__(kWave) FPHO_EVAL_OCCUPANCY void residual_kernel(
         // would hold 4 more registers
         float xb = x, yb = y;
         asm volatile("" : "+v"(xb), "+v"(yb));
-        const double b = minus_value64(rd, g64[off / sizeof(HotGauss)], xb, yb);
+        const double b = minus_value64(
+            rd, g64[__builtin_amdgcn_readfirstlane(H.tag)], xb, yb);
         rd = fabsf(c) > t.tmin ? b : rd - (double)c;
     };
 
-    float hx, hy, hxx, hyy, hxy;   // lane j: Gaussian base + j
+    __shared__ HotGauss rec[kWave];
+    __shared__ float2 rec_lo[CENTRE ? kWave : 1];
+    HotGauss h;   // lane j: Gaussian base + j
+    float2 h_lo = {0.0f, 0.0f};
     auto fetch = [&](int j) {
-        const Global<HotGauss> p = gv + (uint32_t)min(j, ng - 1);
-        hx = p->xcen;
-        hy = p->ycen;
-        hxx = p->sfxx;
-        hyy = p->sfyy;
-        hxy = p->sfxy;
+        const uint32_t i = min(j, ng - 1);
+        h = load_hot(hot + e.gauss_off, i);
+        if (CENTRE) h_lo = {g[i].xcen_lo, g[i].ycen_lo};
     };
     fetch(lane);
     uint64_t *__restrict__ fl = flags + t.flag + k;
     for (int base = 0; base < ng; base += kWave, fl += K) {
         const int j = base + lane;
         const bool hit =
-            j < ng && (cull == 0 || meets(xlo - hx, xhi - hx, ylo - hy, yhi - hy, hxx, hyy, hxy));
-        fetch(j + kWave);   // the next block's, under this block's visits
+            j < ng && (cull == 0 || meets(xlo - h.xcen, xhi - h.xcen, ylo - h.ycen,
+                                          yhi - h.ycen, h.sfxx, h.sfyy, h.sfxy));
         const uint64_t m = __builtin_amdgcn_ballot_w64(hit);
         const int cnt = __builtin_popcountll(m);
-        const uint32_t list = set_first(
-            m, hit, lane, (uint32_t)min(j, ng - 1) * (uint32_t)sizeof(HotGauss));
+        const int rank = rank_in(m);
+        if (hit) {
+            rec[rank] = h;
+            if (CENTRE) rec_lo[rank] = h_lo;
+        }
+        wave_lds_sync();
+        fetch(j + kWave);   // the next block's, under this block's visits
         // bit cnt - 1 - n of act: the n-th visit had a lane inside the cutoff
         // (shifted in through the scalar carry: two additions of act to itself)
         uint32_t act_lo = 0, act_hi = 0;
@@ -834,24 +860,19 @@ __global__ __launch_bounds__(kWave) FPHO_EVAL_OCCUPANCY void residual_kernel(
         };
         int n = 0;
         for (; n + kVisits <= cnt; n += kVisits) {
-            uint32_t off[kVisits];
             HotGauss H[kVisits];
-            float xl[kVisits], yl[kVisits], c[kVisits], top = 0.0f;
-#pragma unroll
-            for (int u = 0; u < kVisits; ++u) off[u] = __builtin_amdgcn_readlane(list, n + u);
+            float2 L[kVisits];
+            float c[kVisits], top = 0.0f;
 #pragma unroll
             for (int u = 0; u < kVisits; ++u) {
-                H[u] = *reinterpret_cast<const HotGauss *>(gh + off[u]);
-                if (CENTRE) {
-                    xl[u] = g[off[u] / sizeof(HotGauss)].xcen_lo;
-                    yl[u] = g[off[u] / sizeof(HotGauss)].ycen_lo;
-                }
+                H[u] = rec[n + u];
+                if (CENTRE) L[u] = rec_lo[n + u];
             }
             __builtin_amdgcn_sched_barrier(0);   // all loads before the first wait
 #pragma unroll
             for (int u = 0; u < kVisits; ++u) {
                 uint64_t in_lanes;
-                c[u] = term(H[u], CENTRE ? xl[u] : 0.0f, CENTRE ? yl[u] : 0.0f, in_lanes);
+                c[u] = term(H[u], L[u], in_lanes);
                 note(in_lanes);
                 if (MIXED) top = fmaxf(top, fabsf(c[u]));
             }
@@ -863,24 +884,23 @@ __global__ __launch_bounds__(kWave) FPHO_EVAL_OCCUPANCY void residual_kernel(
                 for (int u = 0; u < kVisits; ++u) rd -= (double)c[u];
             } else {
 #pragma unroll
-                for (int u = 0; u < kVisits; ++u) subtract_bright(c[u], off[u]);
+                for (int u = 0; u < kVisits; ++u) subtract_bright(c[u], H[u]);
             }
         }
         for (; n < cnt; ++n) {
-            const uint32_t off = __builtin_amdgcn_readlane(list, n);
-            const ImgGauss &G = g[off / sizeof(HotGauss)];
+            const HotGauss H = rec[n];
             uint64_t in_lanes;
-            const float c = term(*reinterpret_cast<const HotGauss *>(gh + off),
-                                 CENTRE ? G.xcen_lo : 0.0f, CENTRE ? G.ycen_lo : 0.0f, in_lanes);
+            const float c = term(H, CENTRE ? rec_lo[n] : float2{0.0f, 0.0f}, in_lanes);
             note(in_lanes);
             if (MIXED)
-                subtract_bright(c, off);
+                subtract_bright(c, H);
             else
                 r -= c;
         }
+        wave_lds_sync();   // before the next block's records
         const uint64_t act = (uint64_t)act_hi << 32 | act_lo;
         const uint64_t word = __builtin_amdgcn_ballot_w64(
-            hit && ((act >> ((cnt - 1 - rank_in(m)) & 63)) & 1));
+            hit && ((act >> ((cnt - 1 - rank) & 63)) & 1));
         if (lane == 0) *fl = word;
     }
     if (!MIXED) rd = (double)r;
@@ -896,10 +916,11 @@ template <int K, bool MIXED, bool CENTRE>
 __global__ __launch_bounds__(kWave) FPHO_EVAL_OCCUPANCY void gradient_kernel(
     const TileDesc *__restrict__ tiles, const int2 *__restrict__ items,
     const ExpDesc *__restrict__ exps, const ImgGauss *__restrict__ gauss,
-    const uint64_t *__restrict__ flags, const double *__restrict__ resid,
+    const HotGauss *__restrict__ hot, const uint64_t *__restrict__ flags,
+    const double *__restrict__ resid,
     const float *__restrict__ weight, float *__restrict__ gpart, double *__restrict__ cpart) {
     const int lane = threadIdx.x;
-    const int2 item = items[xcd_swizzle<kXcdChunk>((int)blockIdx.x, (int)gridDim.x)];
+    const int2 item = items[xcd_rotate((int)blockIdx.x, (int)gridDim.x)];
     const int tile = item.x, s = item.y;
     const TileDesc t = tiles[tile];
     const ExpDesc &e = exps[t.exp];
@@ -948,6 +969,7 @@ __global__ __launch_bounds__(kWave) FPHO_EVAL_OCCUPANCY void gradient_kernel(
     const ImgGauss *__restrict__ g = gauss + e.gauss_off;
     const uint32_t *__restrict__ fl = reinterpret_cast<const uint32_t *>(flags + t.flag);
     const int n_psf = e.n_psf;
+    __shared__ HotGauss rec[kWave];
     SourcePartials src;
     bool touched = false;
     for (int cb = 0; cb < n_psf; cb += kWave) {
@@ -965,27 +987,31 @@ __global__ __launch_bounds__(kWave) FPHO_EVAL_OCCUPANCY void gradient_kernel(
         const int cnt = __builtin_popcountll(m);
         if (cnt == 0) continue;
         touched = true;
-        const uint32_t list = set_first(m, mask != 0, lane, i << 8 | mask);
+        if (mask != 0) {
+            HotGauss h = load_hot(hot + e.gauss_off, i);
+            h.tag = i << 8 | mask;
+            rec[rank_in(m)] = h;
+        }
+        wave_lds_sync();
         for (int n = 0; n < cnt; ++n) {
-            const uint32_t v = __builtin_amdgcn_readlane(list, n);
+            const HotGauss H = rec[n];
+            const uint32_t v = __builtin_amdgcn_readfirstlane(H.tag);
             const ImgGauss &G = g[v >> 8];
-            // read once: left to the slots, each would load them again
-            const float xc = G.xcen, yc = G.ycen;
             const float xcl = CENTRE ? G.xcen_lo : 0.0f, ycl = CENTRE ? G.ycen_lo : 0.0f;
-            const float sfxx = G.sfxx, sfyy = G.sfyy, sfxy = G.sfxy, hcs = G.hcs;
             GradSums q;
 #pragma unroll
             for (int k = 0; k < K; ++k) {
                 if (!(v & (1u << k))) continue;
-                float dx = x[k] - xc, dy = y[k] - yc;
+                float dx = x[k] - H.xcen, dy = y[k] - H.ycen;
                 if (CENTRE) {
                     dx -= xcl;
                     dy -= ycl;
                 }
-                q.add(dx, dy, rr[k], sfxx, sfyy, sfxy, hcs);
+                q.add(dx, dy, rr[k], H.sfxx, H.sfyy, H.sfxy, H.hcs);
             }
             src.add(G, q);
         }
+        wave_lds_sync();   // before the next 64 Gaussians' records
     }
     float *o = gpart + t.part_off + kNParams * s;
     if (touched)
@@ -994,16 +1020,20 @@ __global__ __launch_bounds__(kWave) FPHO_EVAL_OCCUPANCY void gradient_kernel(
         o[lane] = 0.0f;
 }
 
-// The gradient launch's waves: for the q-th tile of the queue, its sources
-// and then its chi2, from items[start[q]].
+// The gradient launch's waves.  A run is the tiles of one exposure that stand
+// together in the queue; its items go source by source (chi2 last), tile by
+// tile, so waves that run together read the same records from the scalar
+// caches (10 bands x 9 exposures, 13 sources: 1071 -> 1023 us a pass against
+// tile by tile).  runs[q]: first item, place in the run and its length.
 __global__ __launch_bounds__(256) void list_items_kernel(
     const TileDesc *__restrict__ tiles, const int32_t *__restrict__ queue,
-    const ExpDesc *__restrict__ exps, const int32_t *__restrict__ start, int32_t n_tiles,
+    const ExpDesc *__restrict__ exps, const int4 *__restrict__ runs, int32_t n_tiles,
     int2 *__restrict__ items) {
     const int q = blockIdx.x * blockDim.x + threadIdx.x;
     if (q >= n_tiles) return;
     const int tile = queue[q], n_src = exps[tiles[tile].exp].n_src;
-    for (int s = 0; s <= n_src; ++s) items[start[q] + s] = make_int2(tile, s);
+    const int4 r = runs[q];
+    for (int s = 0; s <= n_src; ++s) items[r.x + s * r.z + r.y] = make_int2(tile, s);
 }
 
 __global__ void zero_counter_kernel(int32_t *counter) {
@@ -1301,7 +1331,7 @@ static hipError_t launch_eval_k(const EvalArgs &a, hipStream_t stream) {
                            dim3(kWave), 0, stream, a.tiles, a.queue, a.exps, a.gauss, a.gauss64,
                            a.hot, a.slot_boxes, a.flags, a.resid, a.weight, (int32_t)a.cull);
         hipLaunchKernelGGL((gradient_kernel<K, MIXED, CENTRE>), dim3((unsigned)a.n_items),
-                           dim3(kWave), 0, stream, a.tiles, a.items, a.exps, a.gauss, a.flags,
+                           dim3(kWave), 0, stream, a.tiles, a.items, a.exps, a.gauss, a.hot, a.flags,
                            a.resid, a.weight, a.gpart, a.cpart);
         return hipGetLastError();
     }
@@ -1345,11 +1375,11 @@ hipError_t launch_eval(const EvalArgs &a, hipStream_t stream) {
 }
 
 hipError_t launch_list_items(const TileDesc *tiles, const int32_t *queue, const ExpDesc *exps,
-                             const int32_t *start, int64_t n_tiles, int2 *items,
+                             const int4 *runs, int64_t n_tiles, int2 *items,
                              hipStream_t stream) {
     if (n_tiles <= 0) return hipSuccess;
     hipLaunchKernelGGL(list_items_kernel, dim3((unsigned)((n_tiles + 255) / 256)), dim3(256), 0,
-                       stream, tiles, queue, exps, start, (int32_t)n_tiles, items);
+                       stream, tiles, queue, exps, runs, (int32_t)n_tiles, items);
     return hipGetLastError();
 }
 

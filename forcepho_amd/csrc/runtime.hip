@@ -462,36 +462,46 @@ std::vector<int32_t> cost_order(const HostPlan &hp) {
 
 // Whether a plan's pixel pass goes in two launches (residual_kernel,
 // gradient_kernel) instead of one wave per tile.  One wave per tile needs
-// several tiles per wave slot before the waves end together: with 8 or fewer
-// the two launches are faster for every shape measured (us, one wave per
-// tile / two launches: 357 tiles 1012 / 189, 2659 1140 / 420, 13460 1448 /
-// 1041, 26432 2152 / 1955, 52699 2280 / 2174), above it they lose the work
-// that a tile's slots share (106394 tiles 7329 / 7678, 211725 8080 / 8385).
+// many tiles per wave slot before the waves end together: up to 128 slots of 64
+// pixels per wave slot the two launches are faster for every shape measured
+// (us, one wave per tile / two launches: K = 4: 611 tiles 879 / 148, 52699
+// 2209 / 1833, 211725 7987 / 7273; K = 8: 26432 2084 / 1681, 60149 6005 /
+// 5495, 106394 7091 / 6746, with FP64 centres 7578 / 7471); above it they lose
+// the work that a tile's slots share and the gain is gone (K = 8: 206205 12538
+// / 12708, with FP64 centres 13251 / 14392; K = 4: 410508 14244 / 13721).
 // A plan with more than 2^26 flag words (512 MiB: thousands of Gaussians on
-// every pixel) takes one wave per tile too, so the workspace stays bounded.
+// every pixel) takes one wave per tile too, so the workspace stays bounded, and
+// so does one with 2^26 (tile, source) waves, a launch's limit of 2^32 threads.
 bool two_launches(const HostPlan &hp) {
     const int64_t wave_slots = (int64_t)32 * cu_count_cached();
-    return (int64_t)hp.tiles.size() <= 8 * wave_slots && hp.n_flags <= (int64_t)1 << 26;
+    return (int64_t)hp.slot_boxes.size() <= 128 * wave_slots &&
+           hp.n_flags <= (int64_t)1 << 26 &&
+           hp.n_part / kNParams + (int64_t)hp.tiles.size() < (int64_t)1 << 26;
 }
 
 // The wave list and buffers of the two-launch pixel pass.
 int build_two_launches(const HostPlan &hp, const std::vector<int32_t> &queue, Plan &plan) {
-    std::vector<int32_t> start(queue.size());
+    std::vector<int4> runs(queue.size());
     int64_t n_items = 0;
-    for (size_t q = 0; q < queue.size(); ++q) {
-        start[q] = (int32_t)n_items;
-        n_items += hp.exps[hp.tiles[queue[q]].exp].n_src + 1;
+    for (size_t q = 0; q < queue.size();) {
+        const int32_t exp = hp.tiles[queue[q]].exp;
+        size_t end = q;
+        while (end < queue.size() && hp.tiles[queue[end]].exp == exp) ++end;
+        const int32_t len = (int32_t)(end - q);
+        for (int32_t i = 0; i < len; ++i) runs[q + i] = make_int4((int32_t)n_items, i, len, 0);
+        n_items += (int64_t)len * (hp.exps[exp].n_src + 1);
+        q = end;
     }
-    DevVec<int32_t> start_dev;
-    HIP_TRY(start_dev.upload(start.data(), (int64_t)start.size()));
+    DevVec<int4> runs_dev;
+    HIP_TRY(runs_dev.upload(runs.data(), (int64_t)runs.size()));
     HIP_TRY(plan.items.alloc(n_items));
-    HIP_TRY(launch_list_items(plan.tiles.ptr, plan.queue.ptr, plan.exps.ptr, start_dev.ptr,
+    HIP_TRY(launch_list_items(plan.tiles.ptr, plan.queue.ptr, plan.exps.ptr, runs_dev.ptr,
                               (int64_t)queue.size(), plan.items.ptr, nullptr));
     HIP_TRY(plan.hot.alloc(hp.n_gauss));
     HIP_TRY(plan.flags.alloc(hp.n_flags));
     HIP_TRY(plan.resid.alloc((int64_t)hp.slot_boxes.size() * kWave));
     HIP_TRY(plan.weight.alloc((int64_t)hp.slot_boxes.size() * kWave));
-    HIP_TRY(hipStreamSynchronize(nullptr));   // start_dev goes, other streams read the list
+    HIP_TRY(hipStreamSynchronize(nullptr));   // runs_dev goes, other streams read the list
     return FPHO_OK;
 }
 
