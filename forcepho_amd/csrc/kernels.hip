@@ -198,11 +198,6 @@ __global__ __launch_bounds__(kWave) void convert_kernel(
 
 constexpr float kMaskedCoord = 1.0e6f;  // lanes past the tile end: far away
 
-__device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, kWave);
-    return v;
-}
 __device__ __forceinline__ double wave_sum(double v) {
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, kWave);
@@ -303,12 +298,47 @@ struct GradSums {
     }
 };
 
+// v + the value OFF lanes on, in rows of 16 lanes.
+template <int OFF>
+__device__ __forceinline__ float add_ror(float v) {
+    return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x120 | OFF, 0xf,
+                                                          0xf, true));
+}
+
+// Lanes 0-31: a + the value of a 32 lanes on; lanes 32-63: the same of b.
+__device__ __forceinline__ float add_halves(float a, float b) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b),
+                                                    false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
+// Rows 0 and 2: a + the value of a 16 lanes on; rows 1 and 3: the same of b.
+__device__ __forceinline__ float add_rows(float a, float b) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b),
+                                                    false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
+// Row r (of 16 lanes) of the result holds the wave's sum of v_r, its additions
+// paired as a butterfly's over lanes 32, 16, 8, 4, 2, 1 apart.  Four sums share
+// the first two steps' additions and the lanes move in registers: a source's
+// seven sums took 42 LDS shuffles (90 exposures, 13 sources: 955 -> 932 us a
+// pass).
+__device__ __forceinline__ float wave_sum4(float v0, float v1, float v2, float v3) {
+    float v = add_rows(add_halves(v0, v2), add_halves(v1, v3));
+    v = add_ror<8>(v);
+    v = add_ror<4>(v);
+    v = add_ror<2>(v);
+    return add_ror<1>(v);
+}
+
 // A source's 7 partials over the pixels of one lane (position in pixels).
 struct SourcePartials {
     float p0 = 0.f, sx = 0.f, sy = 0.f, p3 = 0.f, p4 = 0.f, p5 = 0.f, p6 = 0.f;
 
     // per-Gaussian epilogue: image-space derivative sums -> 7 partials
-    __device__ __forceinline__ void add(const ImgGauss &G, const GradSums &q) {
+    __device__ __forceinline__ void add(const ImgGauss &G, float sfxx, float sfyy, float sfxy,
+                                        const GradSums &q) {
         const float ke = G.k_e * q.Pe;
         const float gfx = fmaf(G.k_u, q.Peu, fmaf(G.k_axx, q.Pxx, ke));
         const float gfy = fmaf(G.k_u, q.Pea - q.Peu, fmaf(G.k_axx, q.Pyy, ke));
@@ -325,31 +355,23 @@ struct SourcePartials {
         p4 = fmaf(G.dFyy_dPA, gfy, p4);
         p4 = fmaf(G.dFxy_dPA, gfxy, p4);
         // sum e (sF v')_x = sfxx sum e v'x + sfxy sum e v'y (and for y)
-        const float fX = fmaf(G.sfxx, q.X2, G.sfxy * q.Y2);
-        const float fY = fmaf(G.sfxy, q.X2, G.sfyy * q.Y2);
+        const float fX = fmaf(sfxx, q.X2, sfxy * q.Y2);
+        const float fY = fmaf(sfxy, q.X2, sfyy * q.Y2);
         sx = fmaf(G.k_x1, q.X1, fmaf(G.k_x2, fX, sx));
         sy = fmaf(G.k_x1, q.Y1, fmaf(G.k_x2, fY, sy));
     }
 
-    // sum over the wave and write (lane 0); the sky-position derivatives
-    // share the source's CW matrix
+    // sum over the wave and write; the sky-position derivatives share the
+    // source's CW matrix
     __device__ __forceinline__ void write(float *__restrict__ o, const float *__restrict__ CW,
                                           int lane) {
-        p0 = wave_sum(p0);
-        sx = wave_sum(sx);
-        sy = wave_sum(sy);
-        p3 = wave_sum(p3);
-        p4 = wave_sum(p4);
-        p5 = wave_sum(p5);
-        p6 = wave_sum(p6);
-        if (lane == 0) {
-            o[0] = p0;
-            o[1] = fmaf(CW[0], sx, CW[2] * sy);  // dx/dalpha, dy/dalpha
-            o[2] = fmaf(CW[1], sx, CW[3] * sy);  // dx/ddelta, dy/ddelta
-            o[3] = p3;
-            o[4] = p4;
-            o[5] = p5;
-            o[6] = p6;
+        const float u = wave_sum4(sx, p0, p3, p4), v = wave_sum4(sy, p5, p6, 0.0f);
+        if ((lane & 15) == 0) {
+            const int row = lane >> 4;
+            const float dra = fmaf(CW[0], u, CW[2] * v);   // dx/dalpha, dy/dalpha
+            const float ddec = fmaf(CW[1], u, CW[3] * v);  // dx/ddelta, dy/ddelta
+            o[row == 0 ? 1 : row == 1 ? 0 : row + 1] = row == 0 ? dra : u;
+            if (row < 3) o[row == 0 ? 2 : row + 4] = row == 0 ? ddec : v;
         }
     }
 };
@@ -593,7 +615,7 @@ __device__ __forceinline__ void eval_tile(int tile, const TileDesc *__restrict__
                 }
                 q.add(dx, dy, rr[k], sfxx, sfyy, sfxy, hcs);
             }
-            src.add(G, q);
+            src.add(G, sfxx, sfyy, sfxy, q);
           }
         }
         float *o = out + kNParams * s;
@@ -1009,7 +1031,7 @@ __global__ __launch_bounds__(kWave) FPHO_EVAL_OCCUPANCY void gradient_kernel(
                 }
                 q.add(dx, dy, rr[k], H.sfxx, H.sfyy, H.sfxy, H.hcs);
             }
-            src.add(G, q);
+            src.add(G, H.sfxx, H.sfyy, H.sfxy, q);
         }
         wave_lds_sync();   // before the next 64 Gaussians' records
     }
