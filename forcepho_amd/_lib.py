@@ -36,7 +36,7 @@ EXPORTED = [
     "fpho_batch_status", "fpho_batch_free",
     "fpho_spline_create", "fpho_spline_free",
     "fpho_batch_theta_to_proposals_async", "fpho_batch_evaluate_theta_async",
-    "fpho_batch_stack_grad_async",
+    "fpho_batch_stack_grad_async", "fpho_step_async",
 ]
 
 ARRAY_IDS = {"data": 0, "ierr": 1, "xpix": 2, "ypix": 3, "residual": 4}
@@ -59,6 +59,17 @@ class FphoError(RuntimeError):
     def __init__(self, code, msg):
         super().__init__(f"fpho error {code}: {msg}")
         self.code = code
+
+
+class Step(ctypes.Structure):
+    """== fpho_step (include/fpho.h)."""
+    _fields_ = [("n", c_i64),
+                ("z", c_void_p), ("lower", c_void_p), ("range", c_void_p),
+                ("log_range", c_void_p), ("grad_q", c_void_p),
+                ("grad", c_void_p), ("lnjac", c_void_p),
+                ("p", c_void_p), ("eps", c_void_p), ("inv_mass", c_void_p),
+                ("kick", ctypes.c_double),
+                ("p_out", c_void_p), ("z_out", c_void_p), ("q_out", c_void_p)]
 
 
 class PatchDesc(ctypes.Structure):
@@ -124,6 +135,7 @@ def _declare(lib):
         "fpho_batch_theta_to_proposals_async": ([P, P, P, P, P], c_int),
         "fpho_batch_evaluate_theta_async": ([P, P, P, P, P, P, P], c_int),
         "fpho_batch_stack_grad_async": ([P, P, P, P, P, P], c_int),
+        "fpho_step_async": ([ctypes.POINTER(Step), P], c_int),
     }
     for name, (args, res) in sig.items():
         fn = getattr(lib, name)

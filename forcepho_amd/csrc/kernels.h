@@ -75,6 +75,7 @@ hipError_t launch_theta(const SrcDesc *srcs, int64_t n_srcs, const double *theta
 hipError_t launch_stack(const SrcDesc *srcs, int64_t n_srcs, const PatchOut *pouts,
                         int64_t n_patches, const double *chi2, const double *dchi2,
                         double *lnlike, double *grad, hipStream_t stream);
+hipError_t launch_step(const fpho_step &s, hipStream_t stream);
 
 // A batch's current plan as the pixel pass sees it, for the measurement
 // library (libfpho_measure.so); not part of the C ABI.  Rebuilds a stale

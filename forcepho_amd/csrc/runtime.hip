@@ -1319,6 +1319,15 @@ int fpho_batch_stack_grad_async(fpho_batch *b, const double *chi2, const double 
     return FPHO_OK;
 }
 
+int fpho_step_async(const fpho_step *s, void *stream) {
+    if (!s || s->n < 0 || !s->z || !s->lower || !s->range || (s->lnjac && !s->log_range) ||
+        (s->p && (!s->eps || !s->p_out || !(s->grad_q || s->grad))) ||
+        (s->z_out && (!s->p || !s->inv_mass)))
+        return fail(FPHO_E_ARG, "null argument");
+    HIP_TRY(launch_step(*s, (hipStream_t)stream));
+    return FPHO_OK;
+}
+
 }  // extern "C"
 
 // Internal hook of the measurement library (declared in kernels.h, not in the

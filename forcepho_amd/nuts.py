@@ -82,11 +82,7 @@ class NUTS(HMC):
         return (seg(self._velocity(p_start) * r) <= 0) | (seg(self._velocity(p_end) * r) <= 0)
 
     def _leapfrog1(self, z, p, grad, eps):
-        p = p + 0.5 * eps * grad
-        z = z + eps * self._velocity(p)
-        lnp, grad = self.post(z)
-        p = p + 0.5 * eps * grad
-        return z, p, lnp, grad
+        return self.leapfrog(z, p, grad, eps)   # n_steps is 1
 
     def trajectory(self):
         """One NUTS transition of every chain (in place)."""

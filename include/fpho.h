@@ -318,6 +318,29 @@ int fpho_batch_stack_grad_async(fpho_batch *b, const double *chi2_dev,
                                 const double *dchi2_dev, double *lnlike_dev,
                                 double *grad_theta_dev, void *stream);
 
+/* One step of a sampler in the unconstrained space z of parameters bounded by
+ * lower and lower + range (forcepho/model.py:302-368,596-636), over n
+ * parameters, all pointers to device doubles:
+ *   y = sigmoid(z)
+ *   grad_q:  grad = grad_q range y (1 - y) + (1 - 2 y)  (grad may be null);
+ *            without it grad, if any, is read
+ *   lnjac:   lnjac = log_range + ln(y (1 - y))
+ *   p:       p_out = p + kick eps grad
+ *   z_out:   z_out = z + eps inv_mass p_out, and y of it
+ *   q_out:   q_out = lower + y range
+ * A null grad_q, lnjac, p, z_out or q_out leaves its line out.  Outputs may not
+ * overlap inputs. */
+typedef struct fpho_step {
+    int64_t n;
+    const double *z, *lower, *range, *log_range;
+    const double *grad_q;
+    double *grad, *lnjac;
+    const double *p, *eps, *inv_mass;
+    double kick;
+    double *p_out, *z_out, *q_out;
+} fpho_step;
+int fpho_step_async(const fpho_step *step, void *stream);
+
 #ifdef __cplusplus
 }
 #endif
