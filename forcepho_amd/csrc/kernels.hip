@@ -722,13 +722,17 @@ __global__ __launch_bounds__(256) FPHO_EVAL_OCCUPANCY void eval_persistent_kerne
 // exposure is often a whole number of chunks, and without that an XCD would
 // take the same part of every exposure, its crowded middle or its empty edge.
 // Chunks of 128 waves once there are several rows of them, else of 64.
-__device__ __forceinline__ int xcd_rotate(int b, int n) {
+// turn: how far a chunk's waves turn from row to row as well.  Waves are dealt to
+// the CUs in order, so without it the same CU takes the same place of every
+// exposure (turn 29 in the residual launch of 32 exposures of 128^2, 20 sources:
+// 270 -> 249 us a pass; the gradient launch goes source by source and loses 1%).
+__device__ __forceinline__ int xcd_rotate(int b, int n, int turn) {
     const int shift = n >= 1 << 15 ? 7 : 6;   // log2 of the chunk
     const int rows = n >> (shift + 3);
     if (b >= rows << (shift + 3)) return b;
     const int local = b >> 3, row = local >> shift;
     const int xcd = (b + 3 * row) & 7;
-    return (((row << 3) + xcd) << shift) + (local & ((1 << shift) - 1));
+    return (((row << 3) + xcd) << shift) + ((local + turn * row) & ((1 << shift) - 1));
 }
 
 // A pointer known to be to device memory (descriptors hold generic ones), so
@@ -797,7 +801,7 @@ __global__ __launch_bounds__(kWave) FPHO_EVAL_OCCUPANCY void residual_kernel(
     double *__restrict__ resid, float *__restrict__ weight, int32_t cull) {
     constexpr int kVisits = 4;
     const int lane = threadIdx.x;
-    const int wave = xcd_rotate((int)blockIdx.x, (int)gridDim.x);
+    const int wave = xcd_rotate((int)blockIdx.x, (int)gridDim.x, 29);
     const TileDesc t = tiles[queue[wave / K]];
     const int k = wave % K;
     const int npix = t.npix - k * kWave;   // of this slot and the ones after it
@@ -944,7 +948,7 @@ __global__ __launch_bounds__(kWave) FPHO_EVAL_OCCUPANCY void gradient_kernel(
     const double *__restrict__ resid,
     const float *__restrict__ weight, float *__restrict__ gpart, double *__restrict__ cpart) {
     const int lane = threadIdx.x;
-    const int2 item = items[xcd_rotate((int)blockIdx.x, (int)gridDim.x)];
+    const int2 item = items[xcd_rotate((int)blockIdx.x, (int)gridDim.x, 0)];
     const int tile = item.x, s = item.y;
     const TileDesc t = tiles[tile];
     const ExpDesc &e = exps[t.exp];
