@@ -4,9 +4,9 @@
 //   pixels   data, ierr, xpix, ypix, residual : float[npix]  (superpixel order,
 //            exposures concatenated, padding pixels carry ierr = 0)
 //   ImgGauss workspace : one 128-byte record per (exposure, source, psf comp)
-//            written by the convert kernel and read by the pixel kernel with
-//            wave-uniform (scalar) loads; bytes 16-47 are all the residual
-//            pass needs.
+//            written by the convert kernel; the residual pass needs bytes
+//            16-47 only, which the pixel kernels put into LDS, the gradient
+//            epilogue reads the rest with wave-uniform (scalar) loads.
 //   ExpDesc  : one per exposure (batch-global), 128 bytes.
 //   TileDesc : one per wave tile of 64*K pixels of one exposure.
 //   partials : float[n_src*7] per tile + double chi2 per tile; summed in a

@@ -38,8 +38,10 @@ struct EvalArgs {
     int act_words;         // 64-bit activity words per wave (<= kActWordsMax)
 };
 
-// LDS bytes per wave for the pass-1 slot masks, at most (4 waves: 32 KiB).
-constexpr int kMaskCapMax = 8192;
+// LDS bytes per wave for the pass-1 slot masks, at most (4 waves: 24 KiB; with
+// the records and the activity words of as many Gaussians 9 KiB a wave).  8064
+// Gaussians on 12288 tiles: 9862 us with 8192, 8874 with 6144.
+constexpr int kMaskCapMax = 6144;
 constexpr int kActWordsMax = 1024;   // activity bits for 65536 Gaussians per wave
 
 struct SplineView {

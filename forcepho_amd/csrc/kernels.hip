@@ -7,7 +7,7 @@
 //                       partials per source (common_kernel.cc:57-143,
 //                       compute_gaussians_kernel.cu:262-301); one wave per
 //                       tile of 64*K pixels, no float atomics; LDS holds only
-//                       each wave's own slot masks and activity bits.
+//                       each wave's own records, slot masks and activity bits.
 //   residual_kernel, gradient_kernel<K>
 //                       the same in two launches, for small plans: one wave
 //                       per 64-pixel slot, then per (tile, source)
@@ -378,9 +378,44 @@ struct SourcePartials {
     }
 };
 
+// A pointer known to be to device memory (descriptors hold generic ones), so
+// loads take a scalar base and a 32-bit lane offset.
+template <typename T>
+using Global = const T __attribute__((address_space(1))) *;
+template <typename T>
+__device__ __forceinline__ Global<T> global(const T *p) {
+    return (Global<T>)p;
+}
+
+// Set bits of m below this lane.
+__device__ __forceinline__ int rank_in(uint64_t m) {
+    return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
+                                     __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0));
+}
+
+// LDS written by lanes of this wave is visible to its other lanes.
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// The value parameters of Gaussian i; tag: the bits of its peak.
+__device__ __forceinline__ HotGauss load_record(const ImgGauss *__restrict__ g, uint32_t i) {
+    const Global<float4> p = global(reinterpret_cast<const float4 *>(g)) +
+                             sizeof(ImgGauss) / 16 * i + 1;
+    const float4 a = *(const float4 *)p, b = *(const float4 *)(p + 1);
+    return {a.x, a.y, a.z, a.w, b.x, b.y, b.z, __float_as_uint(b.w)};
+}
+
 // Evaluate one wave tile.  `tile` must be wave-uniform (an SGPR value) so
-// every descriptor and Gaussian record load below is a scalar load (the
-// box scan alone reads 64 boxes with one vector load).
+// every descriptor load below is a scalar load.  Bound by VALU issue: a VALU
+// instruction with a scalar operand issues every 4.4 cycles here, one whose
+// operands are all vector registers every 2.6, so both passes take the value
+// parameters of the Gaussians they visit from LDS (64 are put there at once,
+// a visit reads its own with a broadcast) and only the epilogue's constants by
+// scalar loads.  Against scalar loads throughout: 96 patches of 228564 tiles,
+// K = 8, 12440 -> 11730 us (0.35 -> 0.38 VALU instructions a cycle and SIMD);
+// 530123 tiles, K = 4, 19470 -> 17260.
 //   MIXED = true : residual accumulated in FP64; a term whose FP32 value
 //                  exceeds kBrightSigma * sigma of the tile's quietest pixel
 //                  is re-evaluated in FP64 (a wave branch taken only near
@@ -423,7 +458,8 @@ __device__ __forceinline__ void eval_tile(int tile, const TileDesc *__restrict__
                                           float *__restrict__ gpart,
                                           double *__restrict__ cpart, int cull,
                                           uint8_t *__restrict__ amask, int mask_cap,
-                                          uint64_t *__restrict__ act, int act_words) {
+                                          uint64_t *__restrict__ act, int act_words,
+                                          HotGauss *__restrict__ rec) {
     const int lane = threadIdx.x & (kWave - 1);
     const TileDesc t = tiles[tile];
     const ExpDesc &e = exps[t.exp];
@@ -494,40 +530,46 @@ __device__ __forceinline__ void eval_tile(int tile, const TileDesc *__restrict__
                 sm = (1u << K) - 1;
             }
         }
-        uint64_t todo = __builtin_amdgcn_ballot_w64(sm != 0);
+        const uint64_t todo = __builtin_amdgcn_ballot_w64(sm != 0);
+        const int cnt = __builtin_popcountll(todo);
+        if (sm != 0) {
+            HotGauss h = load_record(g, (uint32_t)j);
+            // h.tag: the peak's bits
+            const bool bright = __uint_as_float(h.tag) > tmin;
+            h.tag = (MIXED && bright ? 1u << 31 : 0u) | (uint32_t)lane << 8 | sm;
+            rec[rank_in(todo)] = h;
+        }
+        wave_lds_sync();
         uint64_t active = 0;
-        while (todo) {
-            const int bit = __builtin_ctzll(todo);
-            todo &= todo - 1;
+        for (int n = 0; n < cnt; ++n) {
+            const HotGauss H = rec[n];
+            const uint32_t tag = __builtin_amdgcn_readfirstlane(H.tag);
+            const int bit = (tag >> 8) & 63;
             const int i = base + bit;
-            const uint32_t smi = __builtin_amdgcn_readlane(sm, bit);
             uint32_t m = 0;   // slots with a pixel inside the cutoff (wave-uniform)
-            const float xc = g[i].xcen, yc = g[i].ycen;
             const float xcl = CENTRE ? g[i].xcen_lo : 0.0f, ycl = CENTRE ? g[i].ycen_lo : 0.0f;
-            const float sfxx = g[i].sfxx, sfyy = g[i].sfyy, sfxy = g[i].sfxy;
-            const float hcs = g[i].hcs, ampA = g[i].ampA;
             // a term is bright when |c| > tb: a Gaussian whose peak stays
             // below the tile threshold cannot have one
-            const float tb = g[i].peak > tmin ? tmin : __builtin_huge_valf();
+            const float tb = tag >> 31 ? tmin : __builtin_huge_valf();
 #pragma unroll
             for (int k = 0; k < K; ++k) {
-                if (!(smi & (1u << k))) continue;
-                float dx = x[k] - xc;
-                float dy = y[k] - yc;
+                if (!(tag & (1u << k))) continue;
+                float dx = x[k] - H.xcen;
+                float dy = y[k] - H.ycen;
                 if (CENTRE) {   // the pixel offset from the FP64 centre
                     dx -= xcl;
                     dy -= ycl;
                 }
                 float vx, vy;
-                const float ea = exponent1(dx, dy, sfxx, sfyy, sfxy, vx, vy);   // s E
+                const float ea = exponent1(dx, dy, H.sfxx, H.sfyy, H.sfxy, vx, vy);   // s E
                 const bool in = !(ea < kCutScaled);       // E <= 36 (cutoff)
                 if (__builtin_amdgcn_ballot_w64(in) == 0) continue;
                 m |= 1u << k;
                 {
                     // a lane beyond the cutoff adds an exact zero
                     const float gp = cut_exp(in, ea);
-                    const float h = fmaf(vx, vx, fmaf(vy, vy, hcs));
-                    const float c = ampA * gp * h;
+                    const float h = fmaf(vx, vx, fmaf(vy, vy, H.hcs));
+                    const float c = H.ampA * gp * h;
                     if (MIXED) {
                         if (fabsf(c) > tb) {
                             // keep the FP64 copies of the coordinates inside
@@ -547,6 +589,7 @@ __device__ __forceinline__ void eval_tile(int tile, const TileDesc *__restrict__
             if (i < mask_cap && lane == 0) amask[i] = (uint8_t)m;
         }
         if (lane == 0 && base / kWave < act_words) act[base / kWave] = active;
+        wave_lds_sync();   // before the next 64 Gaussians' records
     }
 
     // pass 2 of this wave reads the masks and activity words of its lane 0
@@ -584,41 +627,44 @@ __device__ __forceinline__ void eval_tile(int tile, const TileDesc *__restrict__
         SourcePartials src;
         const int i0 = s * n_psf;
         bool touched = false;
-        for (int w = i0 / kWave; w <= (i0 + n_psf - 1) / kWave; ++w) {
-          // the source's Gaussians in this word of the activity bits
-          const uint64_t word = w < act_words ? act[w] : ~0ull;
-          const int lo = i0 - w * kWave, hi = i0 + n_psf - w * kWave;   // [lo, hi)
-          uint64_t sel = word;
-          if (lo > 0) sel &= ~0ull << lo;
-          if (hi < kWave) sel &= (1ull << hi) - 1;
-          sel = ((uint64_t)__builtin_amdgcn_readfirstlane((uint32_t)(sel >> 32)) << 32) |
-                (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)sel);
-          while (sel) {
-            const int i = w * kWave + __builtin_ctzll(sel);
-            sel &= sel - 1;
-            const ImgGauss &G = g[i];
-            // slots to evaluate: pass 1's mask, else (past the LDS capacity)
-            // every slot
-            const uint32_t m = i < mask_cap
-                ? (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)amask[i]) : 0xFFu;
+        for (int cb = 0; cb < n_psf; cb += kWave) {
+            // lane l: Gaussian i and the slots to evaluate: pass 1's mask, else
+            // (past the LDS capacity) every slot
+            const bool valid = cb + lane < n_psf;
+            const int i = i0 + (valid ? cb + lane : 0);
+            const int w = i / kWave;
+            const uint64_t word = w < act_words ? act[w] : ~0ull;
+            const bool in = valid && ((word >> (i & (kWave - 1))) & 1);
+            const uint64_t hits = __builtin_amdgcn_ballot_w64(in);
+            const int cnt = __builtin_popcountll(hits);
+            if (cnt == 0) continue;
             touched = true;
-            const float xc = G.xcen, yc = G.ycen;
-            const float xcl = CENTRE ? G.xcen_lo : 0.0f, ycl = CENTRE ? G.ycen_lo : 0.0f;
-            const float sfxx = G.sfxx, sfyy = G.sfyy, sfxy = G.sfxy, hcs = G.hcs;
-            GradSums q;   // over this lane's K pixels
-#pragma unroll
-            for (int k = 0; k < K; ++k) {
-                if (!(m & (1u << k))) continue;
-                float dx = x[k] - xc;
-                float dy = y[k] - yc;
-                if (CENTRE) {
-                    dx -= xcl;
-                    dy -= ycl;
-                }
-                q.add(dx, dy, rr[k], sfxx, sfyy, sfxy, hcs);
+            if (in) {
+                HotGauss h = load_record(g, (uint32_t)i);
+                h.tag = (uint32_t)i << 8 | (i < mask_cap ? amask[i] : 0xFFu);
+                rec[rank_in(hits)] = h;
             }
-            src.add(G, sfxx, sfyy, sfxy, q);
-          }
+            wave_lds_sync();
+            for (int n = 0; n < cnt; ++n) {
+                const HotGauss H = rec[n];
+                const uint32_t v = __builtin_amdgcn_readfirstlane(H.tag);
+                const ImgGauss &G = g[v >> 8];
+                const float xcl = CENTRE ? G.xcen_lo : 0.0f, ycl = CENTRE ? G.ycen_lo : 0.0f;
+                GradSums q;   // over this lane's K pixels
+#pragma unroll
+                for (int k = 0; k < K; ++k) {
+                    if (!(v & (1u << k))) continue;
+                    float dx = x[k] - H.xcen;
+                    float dy = y[k] - H.ycen;
+                    if (CENTRE) {
+                        dx -= xcl;
+                        dy -= ycl;
+                    }
+                    q.add(dx, dy, rr[k], H.sfxx, H.sfyy, H.sfxy, H.hcs);
+                }
+                src.add(G, H.sfxx, H.sfyy, H.sfxy, q);
+            }
+            wave_lds_sync();   // before the next 64 Gaussians' records
         }
         float *o = out + kNParams * s;
         if (!touched) {
@@ -648,9 +694,8 @@ __device__ __forceinline__ int xcd_swizzle(int b, int n) {
 }
 
 // Eight waves per SIMD (the most a SIMD holds) caps the kernels at 64
-// VGPRs (measured at K = 8: 5.7% faster than 6 waves at 76 VGPRs).
-// eval_kernel fits without spills; the persistent kernel at K = 8 spills a
-// few values once per tile, outside every Gaussian loop.
+// VGPRs (measured at K = 8: 5.7% faster than 6 waves at 76 VGPRs); the kernels
+// that keep a tile's residuals spill a few values once per tile.
 #define FPHO_EVAL_OCCUPANCY __attribute__((amdgpu_waves_per_eu(8)))
 
 // Non-persistent: wave w of workgroup b evaluates queue[b*W + w].
@@ -662,17 +707,17 @@ __global__ __launch_bounds__(256) FPHO_EVAL_OCCUPANCY void eval_kernel(
     const int4 *__restrict__ gboxes, const int4 *__restrict__ slot_boxes,
     float *__restrict__ gpart, double *__restrict__ cpart,
     int32_t cull, int32_t mask_cap, int32_t act_words) {
-    extern __shared__ uint64_t lds_words[];
-    uint8_t *lds_mask = reinterpret_cast<uint8_t *>(lds_words);
+    extern __shared__ HotGauss lds_records[];
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int slot = xcd_swizzle<kXcdChunk>((int)blockIdx.x, (int)gridDim.x) *
                      waves_per_group + w;
     if (slot >= n_tiles) return;
     const int tile = __builtin_amdgcn_readfirstlane(queue[slot]);
+    uint8_t *lds_mask = reinterpret_cast<uint8_t *>(lds_records + waves_per_group * kWave);
     eval_tile<K, MIXED, CENTRE>(tile, tiles, exps, gauss, gauss64, gboxes, slot_boxes, gpart, cpart,
                         cull, lds_mask + w * mask_cap, mask_cap,
                         reinterpret_cast<uint64_t *>(lds_mask + waves_per_group * mask_cap) +
-                            w * act_words, act_words);
+                            w * act_words, act_words, lds_records + w * kWave);
 }
 
 // Persistent: every wave pulls tiles from `counter` until the queue is empty.
@@ -685,11 +730,11 @@ __global__ __launch_bounds__(256) FPHO_EVAL_OCCUPANCY void eval_persistent_kerne
     const int4 *__restrict__ gboxes, const int4 *__restrict__ slot_boxes,
     float *__restrict__ gpart, double *__restrict__ cpart,
     int32_t cull, int32_t mask_cap, int32_t act_words) {
-    extern __shared__ uint64_t lds_words[];
-    uint8_t *lds_mask = reinterpret_cast<uint8_t *>(lds_words);
+    extern __shared__ HotGauss lds_records[];
     const int lane = threadIdx.x & (kWave - 1);
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int W = (int)(blockDim.x >> 6);
+    uint8_t *lds_mask = reinterpret_cast<uint8_t *>(lds_records + W * kWave);
     for (;;) {
         int slot = 0;
         if (lane == 0) slot = atomicAdd(counter, 1);
@@ -699,7 +744,7 @@ __global__ __launch_bounds__(256) FPHO_EVAL_OCCUPANCY void eval_persistent_kerne
         eval_tile<K, MIXED, CENTRE>(tile, tiles, exps, gauss, gauss64, gboxes, slot_boxes, gpart,
                             cpart, cull, lds_mask + w * mask_cap, mask_cap,
                             reinterpret_cast<uint64_t *>(lds_mask + W * mask_cap) +
-                                w * act_words, act_words);
+                                w * act_words, act_words, lds_records + w * kWave);
     }
 }
 
@@ -735,15 +780,6 @@ __device__ __forceinline__ int xcd_rotate(int b, int n, int turn) {
     return (((row << 3) + xcd) << shift) + ((local + turn * row) & ((1 << shift) - 1));
 }
 
-// A pointer known to be to device memory (descriptors hold generic ones), so
-// loads take a scalar base and a 32-bit lane offset.
-template <typename T>
-using Global = const T __attribute__((address_space(1))) *;
-template <typename T>
-__device__ __forceinline__ Global<T> global(const T *p) {
-    return (Global<T>)p;
-}
-
 // False only if no point of the box [xlo, xhi] x [ylo, yhi] (relative to the
 // Gaussian's centre) lies inside its cutoff ellipse E <= 36.  The smallest E
 // of a box that does not hold the centre is on an edge that faces the centre;
@@ -762,18 +798,6 @@ __device__ __forceinline__ bool meets(float xlo, float xhi, float ylo, float yhi
     const float k = sfxx * sfyy;
     const float wide = k * __builtin_amdgcn_rcpf(fmaxf(fmaf(-sfxy, sfxy, k), 0.0f));
     return !(fmaxf(ea, eb) < kCutScaled * fmaf(4e-6f, wide, 1.001f));
-}
-
-// Set bits of m below this lane.
-__device__ __forceinline__ int rank_in(uint64_t m) {
-    return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
-                                     __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0));
-}
-
-// LDS written by lanes of this wave is visible to its other lanes.
-__device__ __forceinline__ void wave_lds_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-    __builtin_amdgcn_wave_barrier();
 }
 
 // The record of Gaussian i, tagged with i (two 16-byte loads).
@@ -1404,8 +1428,9 @@ static hipError_t launch_eval_k(const EvalArgs &a, hipStream_t stream) {
         return hipGetLastError();
     }
     const int W = a.waves_per_group;
-    // per wave: the slot mask bytes, then the activity words
-    const size_t lds = (size_t)W * ((size_t)a.mask_cap + 8 * (size_t)a.act_words);
+    // per wave: 64 records, the slot mask bytes, then the activity words
+    const size_t lds = (size_t)W * (kWave * sizeof(HotGauss) + (size_t)a.mask_cap +
+                                    8 * (size_t)a.act_words);
     if (a.persistent) {
         hipLaunchKernelGGL(zero_counter_kernel, dim3(1), dim3(64), 0, stream, a.counter);
         hipLaunchKernelGGL((eval_persistent_kernel<K, MIXED, CENTRE>), dim3((unsigned)a.grid),

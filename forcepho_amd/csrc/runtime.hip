@@ -462,19 +462,20 @@ std::vector<int32_t> cost_order(const HostPlan &hp) {
 
 // Whether a plan's pixel pass goes in two launches (residual_kernel,
 // gradient_kernel) instead of one wave per tile.  One wave per tile needs
-// many tiles per wave slot before the waves end together: up to 128 slots of 64
-// pixels per wave slot the two launches are faster for every shape measured
-// (us, one wave per tile / two launches: K = 4: 611 tiles 879 / 148, 52699
-// 2209 / 1833, 211725 7987 / 7273; K = 8: 26432 2084 / 1681, 60149 6005 /
-// 5495, 106394 7091 / 6746, with FP64 centres 7578 / 7471); above it they lose
-// the work that a tile's slots share and the gain is gone (K = 8: 206205 12538
-// / 12708, with FP64 centres 13251 / 14392; K = 4: 410508 14244 / 13721).
+// many tiles per wave slot before the waves end together; up to 10 the two
+// launches are faster (us, one wave per tile / two launches, in brackets with
+// FP64 centres.  K = 8: 16419 tiles 1860 / 1413 (1974 / 1522), 55694 3497 / 3166
+// (3654 / 3494), 75042 4843 / 4478 (4979 / 4968); K = 4: 611 879 / 148, 52699
+// 1998 / 1797 (2111 / 1960)), above it the work that a tile's slots share
+// counts for more (K = 8: 106394 7072 / 6639 (7288 / 7420), 146737 9119 / 9041
+// (9381 / 10056); K = 4: 110912 3476 / 3399 (3677 / 3729), 211725 7089 / 7228
+// (7607 / 8137)).
 // A plan with more than 2^26 flag words (512 MiB: thousands of Gaussians on
 // every pixel) takes one wave per tile too, so the workspace stays bounded, and
 // so does one with 2^26 (tile, source) waves, a launch's limit of 2^32 threads.
 bool two_launches(const HostPlan &hp) {
     const int64_t wave_slots = (int64_t)32 * cu_count_cached();
-    return (int64_t)hp.slot_boxes.size() <= 128 * wave_slots &&
+    return (int64_t)hp.tiles.size() <= 10 * wave_slots &&
            hp.n_flags <= (int64_t)1 << 26 &&
            hp.n_part / kNParams + (int64_t)hp.tiles.size() < (int64_t)1 << 26;
 }
