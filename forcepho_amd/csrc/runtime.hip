@@ -79,6 +79,13 @@ struct DevVec {
     }
 };
 
+// Part of a device buffer.
+template <typename T>
+struct Span {
+    T *ptr = nullptr;
+    int64_t n = 0;
+};
+
 // Page-locked host buffer (hipHostMalloc): copies from and to it run
 // asynchronously, without a staging copy inside the runtime.
 template <typename T>
@@ -152,28 +159,37 @@ int cu_count_cached() {
 
 // Tile plan over one or more patches (single-patch drop-in or batch).
 struct Plan {
-    DevVec<ExpDesc> exps;
-    DevVec<TileDesc> tiles;
-    DevVec<int32_t> queue;
-    DevVec<OutDesc> outs;
-    DevVec<ImgGauss> gauss;
-    DevVec<ImgGauss64> gauss64;
-    DevVec<int4> gboxes;
+    // all in one allocation: a plan of its ~20 buffers took as long to allocate
+    // as a small patch takes to evaluate five times
+    DevVec<unsigned char> arena;
+    Span<ExpDesc> exps;
+    Span<TileDesc> tiles;
+    Span<int4> slot_boxes;
+    Span<int32_t> queue;
+    Span<OutDesc> outs;
+    Span<SrcDesc> srcs;
+    Span<PatchOut> pouts;
+    Span<int32_t> counter;
+    Span<uint32_t> status;        // FPHO_STATUS_* bits of the plan's kernels
+    Span<ImgGauss> gauss;
+    Span<ImgGauss64> gauss64;
+    Span<int4> gboxes;
     // two-launch pixel pass (empty unless the plan uses it)
-    DevVec<HotGauss> hot;
-    DevVec<int2> items;
-    DevVec<uint64_t> flags;
-    DevVec<double> resid;
-    DevVec<float> weight;
-    DevVec<int4> slot_boxes;
-    DevVec<float> gpart;
-    DevVec<double> cpart;
-    DevVec<int32_t> counter;
-    DevVec<uint32_t> status;        // FPHO_STATUS_* bits of the plan's kernels
-    DevVec<double> dchi2_tmp;       // single patch: dchi2 before the compat Response layout
-    DevVec<SrcDesc> srcs;
-    DevVec<PatchOut> pouts;
-    DevVec<Source64> src64;         // batch: FP64 source records of the theta path
+    Span<int4> runs;
+    Span<int2> items;
+    Span<HotGauss> hot;
+    Span<uint64_t> flags;
+    Span<double> resid;
+    Span<float> weight;
+    Span<float> gpart;
+    Span<double> cpart;
+    Span<Source64> src64;         // batch: FP64 source records of the theta path
+    // single patch: the synchronous drop-in's proposal and results (chi2
+    // [n_bands], then dchi2 [n_bands][n_sources][7]), and dchi2 before the
+    // compat Response layout
+    Span<fpho_source> prop;
+    Span<double> out;
+    Span<double> dchi2_tmp;
     int64_t n_exp = 0, n_tiles = 0, n_outs = 0, n_gauss = 0, n_srcs = 0, n_patches = 0;
     int64_t n_pairs = 0, npix = 0, n_part = 0;
     int32_t max_ng = 0;  // most image Gaussians of one exposure
@@ -216,13 +232,9 @@ struct fpho_patch {
     int precision = kPrecMixed;
     Plan plan;
     uint64_t plan_generation = 0;
-    // staging for the synchronous drop-in: the proposal, and chi2 [n_bands]
-    // followed by dchi2 [n_bands][n_sources][7] in one buffer, so a call
-    // makes one copy each way from page-locked memory and one wait
-    DevVec<fpho_source> prop_dev;
-    DevVec<double> out_dev;
-    PinnedVec<fpho_source> prop_host;
-    PinnedVec<double> out_host;
+    // the synchronous drop-in's proposal and results in page-locked memory, so
+    // a call makes one copy each way and one wait
+    PinnedVec<double> io_host;
 };
 
 struct fpho_batch {
@@ -480,9 +492,11 @@ bool two_launches(const HostPlan &hp) {
            hp.n_part / kNParams + (int64_t)hp.tiles.size() < (int64_t)1 << 26;
 }
 
-// The wave list and buffers of the two-launch pixel pass.
-int build_two_launches(const HostPlan &hp, const std::vector<int32_t> &queue, Plan &plan) {
-    std::vector<int4> runs(queue.size());
+// Where the waves of each tile of the queue stand in the two-launch pixel
+// pass's list (launch_list_items); returns how many there are.
+int64_t item_runs(const HostPlan &hp, const std::vector<int32_t> &queue,
+                  std::vector<int4> &runs) {
+    runs.resize(queue.size());
     int64_t n_items = 0;
     for (size_t q = 0; q < queue.size();) {
         const int32_t exp = hp.tiles[queue[q]].exp;
@@ -493,16 +507,54 @@ int build_two_launches(const HostPlan &hp, const std::vector<int32_t> &queue, Pl
         n_items += (int64_t)len * (hp.exps[exp].n_src + 1);
         q = end;
     }
-    DevVec<int4> runs_dev;
-    HIP_TRY(runs_dev.upload(runs.data(), (int64_t)runs.size()));
-    HIP_TRY(plan.items.alloc(n_items));
-    HIP_TRY(launch_list_items(plan.tiles.ptr, plan.queue.ptr, plan.exps.ptr, runs_dev.ptr,
-                              (int64_t)queue.size(), plan.items.ptr, nullptr));
-    HIP_TRY(plan.hot.alloc(hp.n_gauss));
-    HIP_TRY(plan.flags.alloc(hp.n_flags));
-    HIP_TRY(plan.resid.alloc((int64_t)hp.slot_boxes.size() * kWave));
-    HIP_TRY(plan.weight.alloc((int64_t)hp.slot_boxes.size() * kWave));
-    HIP_TRY(hipStreamSynchronize(nullptr));   // runs_dev goes, other streams read the list
+    return n_items;
+}
+
+int64_t align256(int64_t x) { return (x + 255) & ~(int64_t)255; }
+
+// The parts of a plan's allocation, each 256-byte aligned.
+struct Layout {
+    struct Part {
+        void **ptr;
+        const void *host;   // copied to the device, if any
+        int64_t at, bytes;
+    };
+    std::vector<Part> parts;
+    int64_t bytes = 0, uploaded = 0;   // uploaded: bytes up to the last part with data
+
+    template <typename T>
+    void add(Span<T> &span, int64_t count, const T *host = nullptr) {
+        span.ptr = nullptr;
+        span.n = std::max<int64_t>(count, 0);
+        if (count <= 0) return;
+        const int64_t n = (int64_t)sizeof(T) * count;
+        parts.push_back({(void **)&span.ptr, host, bytes, n});
+        if (host) uploaded = bytes + n;
+        bytes = align256(bytes + n);
+    }
+};
+
+// Allocate, place and fill.  Buffers that work on any stream may still read are
+// not touched before the device is idle (hipFree waits for it too).
+int place_plan(const Layout &layout, Plan &plan) {
+    if (layout.bytes > plan.arena.n || layout.bytes < plan.arena.n / 4)
+        HIP_TRY(plan.arena.alloc(layout.bytes));
+    else
+        HIP_TRY(hipDeviceSynchronize());
+    unsigned char *base = plan.arena.ptr;
+    for (const Layout::Part &part : layout.parts) *part.ptr = base + part.at;
+    // up to 1 MiB of descriptors goes in one copy; more is not worth gathering
+    if (layout.uploaded <= 1 << 20) {
+        std::vector<unsigned char> stage((size_t)layout.uploaded);
+        for (const Layout::Part &part : layout.parts)
+            if (part.host) std::memcpy(stage.data() + part.at, part.host, (size_t)part.bytes);
+        HIP_TRY(hipMemcpy(base, stage.data(), stage.size(), hipMemcpyHostToDevice));
+        return FPHO_OK;
+    }
+    for (const Layout::Part &part : layout.parts)
+        if (part.host)
+            HIP_TRY(hipMemcpy(base + part.at, part.host, (size_t)part.bytes,
+                              hipMemcpyHostToDevice));
     return FPHO_OK;
 }
 
@@ -532,38 +584,47 @@ int build_plan(const std::vector<fpho_patch *> &patches, const fpho_launch &laun
     // ties keep canonical order, so tiles of one exposure stay adjacent.
     const std::vector<int32_t> queue = cost_order(hp);
 
-    HIP_TRY(plan.exps.upload(hp.exps.data(), (int64_t)hp.exps.size()));
-    HIP_TRY(plan.tiles.upload(hp.tiles.data(), (int64_t)hp.tiles.size()));
-    HIP_TRY(plan.slot_boxes.upload(hp.slot_boxes.data(), (int64_t)hp.slot_boxes.size()));
-    HIP_TRY(plan.queue.upload(queue.data(), (int64_t)queue.size()));
-    HIP_TRY(plan.outs.upload(hp.outs.data(), (int64_t)hp.outs.size()));
-    HIP_TRY(plan.srcs.upload(hp.srcs.data(), (int64_t)hp.srcs.size()));
-    HIP_TRY(plan.pouts.upload(hp.pouts.data(), (int64_t)hp.pouts.size()));
-    HIP_TRY(plan.gauss.alloc(hp.n_gauss));
-    HIP_TRY(plan.gauss64.alloc(hp.n_gauss));
-    HIP_TRY(plan.gboxes.alloc(hp.n_gauss));
-    plan.hot.release();
-    plan.items.release();
-    plan.flags.release();
-    plan.resid.release();
-    plan.weight.release();
-    if (two_launches(hp)) {
-        const int rc = build_two_launches(hp, queue, plan);
-        if (rc) return rc;
+    const int64_t n_tiles = (int64_t)hp.tiles.size();
+    const int64_t n_slots = (int64_t)hp.slot_boxes.size();
+    const bool two = two_launches(hp);
+    std::vector<int4> runs;
+    const int64_t n_items = two ? item_runs(hp, queue, runs) : 0;
+    const int32_t zero = 0;
+    const uint32_t no_status = 0;
+    Layout layout;
+    layout.add(plan.exps, (int64_t)hp.exps.size(), hp.exps.data());
+    layout.add(plan.tiles, n_tiles, hp.tiles.data());
+    layout.add(plan.slot_boxes, n_slots, hp.slot_boxes.data());
+    layout.add(plan.queue, (int64_t)queue.size(), queue.data());
+    layout.add(plan.outs, (int64_t)hp.outs.size(), hp.outs.data());
+    layout.add(plan.srcs, (int64_t)hp.srcs.size(), hp.srcs.data());
+    layout.add(plan.pouts, (int64_t)hp.pouts.size(), hp.pouts.data());
+    layout.add(plan.counter, 1, &zero);
+    layout.add(plan.status, 1, &no_status);
+    layout.add(plan.runs, (int64_t)runs.size(), runs.data());
+    layout.add(plan.gauss, hp.n_gauss);
+    layout.add(plan.gauss64, hp.n_gauss);
+    layout.add(plan.gboxes, hp.n_gauss);
+    layout.add(plan.items, n_items);
+    layout.add(plan.hot, two ? hp.n_gauss : 0);
+    layout.add(plan.flags, two ? hp.n_flags : 0);
+    layout.add(plan.resid, two ? n_slots * kWave : 0);
+    layout.add(plan.weight, two ? n_slots * kWave : 0);
+    layout.add(plan.gpart, std::max<int64_t>(hp.n_part, 1));
+    layout.add(plan.cpart, std::max<int64_t>(n_tiles, 1));
+    layout.add(plan.src64, std::max<int64_t>((int64_t)hp.srcs.size(), 1));
+    const fpho_patch *one = patches.size() == 1 ? patches[0] : nullptr;
+    const int64_t nd = one ? (int64_t)one->n_bands * one->n_sources * kNParams : 0;
+    layout.add(plan.prop, one ? one->n_sources : 0);
+    layout.add(plan.out, one ? one->n_bands + nd : 0);
+    layout.add(plan.dchi2_tmp, nd);
+    const int rc = place_plan(layout, plan);
+    if (rc) return rc;
+    if (n_items > 0) {
+        HIP_TRY(launch_list_items(plan.tiles.ptr, plan.queue.ptr, plan.exps.ptr, plan.runs.ptr,
+                                  n_tiles, plan.items.ptr, nullptr));
+        HIP_TRY(hipStreamSynchronize(nullptr));   // other streams read the list
     }
-    HIP_TRY(plan.gpart.alloc(std::max<int64_t>(hp.n_part, 1)));
-    HIP_TRY(plan.cpart.alloc(std::max<int64_t>((int64_t)hp.tiles.size(), 1)));
-    HIP_TRY(plan.counter.alloc(1));
-    HIP_TRY(hipMemset(plan.counter.ptr, 0, sizeof(int32_t)));
-    HIP_TRY(plan.status.alloc(1));
-    HIP_TRY(hipMemset(plan.status.ptr, 0, sizeof(uint32_t)));
-    if (patches.size() == 1) {
-        const fpho_patch *p = patches[0];
-        HIP_TRY(plan.dchi2_tmp.alloc((int64_t)p->n_bands * p->n_sources * kNParams));
-    } else {
-        plan.dchi2_tmp.release();
-    }
-    HIP_TRY(plan.src64.alloc(std::max<int64_t>((int64_t)hp.srcs.size(), 1)));
     plan.n_exp = (int64_t)hp.exps.size();
     plan.n_tiles = (int64_t)hp.tiles.size();
     plan.n_outs = (int64_t)hp.outs.size();
@@ -740,8 +801,6 @@ int scratch_address(int device, unsigned char **out) {
     return FPHO_OK;
 }
 
-int64_t align256(int64_t x) { return (x + 255) & ~(int64_t)255; }
-
 // True when `stream` is capturing a graph (plans are not rebuilt then: a
 // rebuild allocates and copies synchronously).
 bool capturing(hipStream_t stream) {
@@ -817,26 +876,24 @@ int check_proposal_host(const fpho_patch *p, const fpho_source *prop) {
 
 // Synchronous evaluation through the patch's page-locked staging: host
 // proposal in, chi2 [n_bands] and dchi2 [n_bands][n_sources][7] (double) out
-// in out_host.
-int evaluate_sync(fpho_patch *p, const fpho_source *prop) {
+// at *out_host.
+int evaluate_sync(fpho_patch *p, const fpho_source *prop, double **out_host) {
     int rc = check_proposal_host(p, prop);
     if (rc) return rc;
     rc = ensure_patch_plan(p, nullptr);
     if (rc) return rc;
-    const int64_t nd = (int64_t)p->n_bands * p->n_sources * kNParams;
-    const int64_t nout = p->n_bands + nd;
-    if (p->prop_dev.n < p->n_sources) HIP_TRY(p->prop_dev.alloc(p->n_sources));
-    if (p->out_dev.n < nout) HIP_TRY(p->out_dev.alloc(nout));
-    if (p->prop_host.n < p->n_sources) HIP_TRY(p->prop_host.alloc(p->n_sources));
-    if (p->out_host.n < nout) HIP_TRY(p->out_host.alloc(nout));
-    std::memcpy(p->prop_host.ptr, prop, sizeof(fpho_source) * p->n_sources);
-    HIP_TRY(hipMemcpyAsync(p->prop_dev.ptr, p->prop_host.ptr,
-                           sizeof(fpho_source) * p->n_sources, hipMemcpyHostToDevice, nullptr));
-    rc = run_plan(p->plan, p->status.ptr, p->prop_dev.ptr, p->out_dev.ptr,
-                  p->out_dev.ptr + p->n_bands,
-                  nullptr);
+    Plan &plan = p->plan;
+    const int64_t prop_bytes = align256((int64_t)sizeof(fpho_source) * plan.prop.n);
+    const int64_t need = prop_bytes / (int64_t)sizeof(double) + plan.out.n;
+    if (p->io_host.n < need) HIP_TRY(p->io_host.alloc(need));
+    std::memcpy(p->io_host.ptr, prop, sizeof(fpho_source) * plan.prop.n);
+    HIP_TRY(hipMemcpyAsync(plan.prop.ptr, p->io_host.ptr, sizeof(fpho_source) * plan.prop.n,
+                           hipMemcpyHostToDevice, nullptr));
+    rc = run_plan(plan, p->status.ptr, plan.prop.ptr, plan.out.ptr,
+                  plan.out.ptr + p->n_bands, nullptr);
     if (rc) return rc;
-    HIP_TRY(hipMemcpyAsync(p->out_host.ptr, p->out_dev.ptr, sizeof(double) * nout,
+    *out_host = p->io_host.ptr + prop_bytes / (int64_t)sizeof(double);
+    HIP_TRY(hipMemcpyAsync(*out_host, plan.out.ptr, sizeof(double) * plan.out.n,
                            hipMemcpyDeviceToHost, nullptr));
     HIP_TRY(hipStreamSynchronize(nullptr));
     return FPHO_OK;
@@ -1042,11 +1099,12 @@ int fpho_patch_free(fpho_patch *p) {
 
 int fpho_evaluate(fpho_patch *p, const fpho_source *prop, double *chi2, float *dchi2) {
     if (!p || !prop || !chi2 || !dchi2) return fail(FPHO_E_ARG, "null argument");
-    const int rc = evaluate_sync(p, prop);
+    double *out = nullptr;
+    const int rc = evaluate_sync(p, prop, &out);
     if (rc) return rc;
     const int64_t nd = (int64_t)p->n_bands * p->n_sources * kNParams;
-    std::memcpy(chi2, p->out_host.ptr, sizeof(double) * p->n_bands);
-    for (int64_t i = 0; i < nd; ++i) dchi2[i] = (float)p->out_host.ptr[p->n_bands + i];
+    std::memcpy(chi2, out, sizeof(double) * p->n_bands);
+    for (int64_t i = 0; i < nd; ++i) dchi2[i] = (float)out[p->n_bands + i];
     return FPHO_OK;
 }
 
@@ -1114,12 +1172,13 @@ int fpho_evaluate_response(fpho_patch *p, const fpho_source *prop, double *chi2,
     if (p->n_sources > FPHO_MAXSOURCES)
         return fail(FPHO_E_LIMIT, "%d sources do not fit the Response layout (MAXSOURCES %d)",
                     p->n_sources, FPHO_MAXSOURCES);
-    const int rc = evaluate_sync(p, prop);
+    double *out = nullptr;
+    const int rc = evaluate_sync(p, prop, &out);
     if (rc) return rc;
-    std::memcpy(chi2, p->out_host.ptr, sizeof(double) * p->n_bands);
+    std::memcpy(chi2, out, sizeof(double) * p->n_bands);
     const int nw = p->n_sources * kNParams;
     for (int b = 0; b < p->n_bands; ++b) {
-        const double *src = p->out_host.ptr + p->n_bands + (int64_t)b * nw;
+        const double *src = out + p->n_bands + (int64_t)b * nw;
         for (int j = 0; j < FPHO_MAXSOURCES * kNParams; ++j)
             resp[b].dchi2_dparam[j] = j < nw ? (float)src[j] : 0.0f;
     }
