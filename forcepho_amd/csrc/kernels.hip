@@ -760,8 +760,8 @@ __global__ __launch_bounds__(256) FPHO_EVAL_OCCUPANCY void eval_persistent_kerne
 //
 // What bounds it: VALU issue, and on small plans the serial chain of the
 // heaviest wave.  Measured (us, one wave per tile -> two launches): 16 tiles
-// of 54 Gaussians 58 -> 29; 2048 tiles of 720 535 -> 260; 6144 tiles of 2160
-// 1440 -> 980; 575 tiles of up to 1620 (four patches) 882 -> 125.
+// of 54 Gaussians 58 -> 28; 2048 tiles of 720 535 -> 247; 6144 tiles of 2160
+// 1440 -> 905; 611 tiles of up to 1620 (four patches) 882 -> 134.
 
 // xcd_swizzle with the XCDs' chunks moved on by three from row to row: an
 // exposure is often a whole number of chunks, and without that an XCD would

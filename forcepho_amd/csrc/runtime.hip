@@ -178,9 +178,11 @@ struct Plan {
     Span<int4> runs;
     Span<int2> items;
     Span<HotGauss> hot;
-    Span<uint64_t> flags;
-    Span<double> resid;
-    Span<float> weight;
+    // its workspace (flags, residuals, weights: 12 bytes a pixel and more),
+    // held by plans that are evaluated stream ordered; synchronous evaluations
+    // share one per device
+    DevVec<unsigned char> work;
+    int64_t n_flags = 0, n_slots = 0;
     Span<float> gpart;
     Span<double> cpart;
     Span<Source64> src64;         // batch: FP64 source records of the theta path
@@ -534,6 +536,12 @@ struct Layout {
     }
 };
 
+// Bytes of a plan's two-launch workspace; 0 for one wave per tile.
+int64_t work_bytes(const Plan &plan) {
+    return align256((int64_t)sizeof(uint64_t) * plan.n_flags) +
+           plan.n_slots * kWave * (int64_t)(sizeof(double) + sizeof(float));
+}
+
 // Allocate, place and fill.  Buffers that work on any stream may still read are
 // not touched before the device is idle (hipFree waits for it too).
 int place_plan(const Layout &layout, Plan &plan) {
@@ -607,9 +615,6 @@ int build_plan(const std::vector<fpho_patch *> &patches, const fpho_launch &laun
     layout.add(plan.gboxes, hp.n_gauss);
     layout.add(plan.items, n_items);
     layout.add(plan.hot, two ? hp.n_gauss : 0);
-    layout.add(plan.flags, two ? hp.n_flags : 0);
-    layout.add(plan.resid, two ? n_slots * kWave : 0);
-    layout.add(plan.weight, two ? n_slots * kWave : 0);
     layout.add(plan.gpart, std::max<int64_t>(hp.n_part, 1));
     layout.add(plan.cpart, std::max<int64_t>(n_tiles, 1));
     layout.add(plan.src64, std::max<int64_t>((int64_t)hp.srcs.size(), 1));
@@ -618,8 +623,12 @@ int build_plan(const std::vector<fpho_patch *> &patches, const fpho_launch &laun
     layout.add(plan.prop, one ? one->n_sources : 0);
     layout.add(plan.out, one ? one->n_bands + nd : 0);
     layout.add(plan.dchi2_tmp, nd);
+    plan.n_flags = two ? hp.n_flags : 0;
+    plan.n_slots = two ? n_slots : 0;
     const int rc = place_plan(layout, plan);
     if (rc) return rc;
+    // (the device is idle)
+    if (work_bytes(plan) > plan.work.n || work_bytes(plan) < plan.work.n / 4) plan.work.release();
     if (n_items > 0) {
         HIP_TRY(launch_list_items(plan.tiles.ptr, plan.queue.ptr, plan.exps.ptr, plan.runs.ptr,
                                   n_tiles, plan.items.ptr, nullptr));
@@ -672,8 +681,19 @@ struct PlanPtrs {
     hipEvent_t *ev = nullptr;
 };
 
-PlanPtrs plan_ptrs(Plan &plan, uint32_t *status) {
+// `work`: the two-launch workspace; without one the pixel pass takes one wave
+// per tile (same results).
+PlanPtrs plan_ptrs(Plan &plan, uint32_t *status, unsigned char *work) {
     PlanPtrs q;
+    if (work != nullptr) {
+        q.hot = plan.hot.ptr;
+        q.items = plan.items.ptr;
+        q.n_items = plan.items.n;
+        q.flags = reinterpret_cast<uint64_t *>(work);
+        q.resid = reinterpret_cast<double *>(
+            work + align256((int64_t)sizeof(uint64_t) * plan.n_flags));
+        q.weight = reinterpret_cast<float *>(q.resid + plan.n_slots * kWave);
+    }
     q.exps = plan.exps.ptr;
     q.tiles = plan.tiles.ptr;
     q.queue = plan.queue.ptr;
@@ -682,12 +702,6 @@ PlanPtrs plan_ptrs(Plan &plan, uint32_t *status) {
     q.gauss = plan.gauss.ptr;
     q.gauss64 = plan.gauss64.ptr;
     q.gboxes = plan.gboxes.ptr;
-    q.hot = plan.hot.ptr;
-    q.items = plan.items.ptr;
-    q.flags = plan.flags.ptr;
-    q.resid = plan.resid.ptr;
-    q.weight = plan.weight.ptr;
-    q.n_items = plan.items.n;
     q.gpart = plan.gpart.ptr;
     q.cpart = plan.cpart.ptr;
     q.counter = plan.counter.ptr;
@@ -737,7 +751,9 @@ EvalArgs eval_args(const PlanPtrs &q) {
     return a;
 }
 
-EvalArgs eval_args(Plan &plan) { return eval_args(plan_ptrs(plan, plan.status.ptr)); }
+EvalArgs eval_args(Plan &plan) {
+    return eval_args(plan_ptrs(plan, plan.status.ptr, plan.work.ptr));
+}
 
 // convert -> pixel pass -> reduce on `stream`
 template <typename Src>
@@ -759,9 +775,9 @@ int run_ptrs(const PlanPtrs &q, const Src *props, double *chi2, double *dchi2,
 // A single patch's plan reports into the patch's status word, a batch's
 // into the plan's.
 template <typename Src>
-int run_plan(Plan &plan, uint32_t *status, const Src *props, double *chi2, double *dchi2,
-             hipStream_t stream) {
-    return run_ptrs(plan_ptrs(plan, status), props, chi2, dchi2, stream);
+int run_plan(Plan &plan, uint32_t *status, unsigned char *work, const Src *props, double *chi2,
+             double *dchi2, hipStream_t stream) {
+    return run_ptrs(plan_ptrs(plan, status, work), props, chi2, dchi2, stream);
 }
 
 }  // namespace
@@ -809,6 +825,36 @@ bool capturing(hipStream_t stream) {
     return st != hipStreamCaptureStatusNone;
 }
 
+// The plan's own two-launch workspace, allocated at its first stream-ordered
+// evaluation; null (one wave per tile) where it is not to be had.
+unsigned char *own_work(Plan &plan, hipStream_t stream) {
+    const int64_t bytes = work_bytes(plan);
+    if (bytes == 0) return nullptr;
+    if (plan.work.n < bytes) {
+        if (capturing(stream)) return nullptr;
+        if (plan.work.alloc(bytes) != hipSuccess) {
+            (void)hipGetLastError();
+            return nullptr;
+        }
+    }
+    return plan.work.ptr;
+}
+
+// The two-launch workspace of synchronous evaluations, which all run on the
+// null stream: one per device, at most half as large again as the largest patch
+// evaluated needs (a plan of two launches has at most 320 tiles per CU and 2^26
+// flag words: 1 GiB), freed with the device's last patch.  The lock covers a call's launches, so
+// calls of several threads follow each other on the stream.
+struct SharedWork {
+    std::mutex mu;
+    DevVec<unsigned char> buf;
+    int64_t patches = 0;
+};
+SharedWork *shared_work(int device) {
+    static SharedWork *const all = new SharedWork[kScratchDevices];   // never destroyed
+    return all + std::min(std::max(device, 0), kScratchDevices - 1);
+}
+
 int ensure_patch_plan(fpho_patch *p, hipStream_t stream) {
     if (p->plan.valid && p->plan_generation == p->generation) return FPHO_OK;
     if (capturing(stream))
@@ -841,6 +887,7 @@ int ensure_batch_plan(fpho_batch *b, hipStream_t stream) {
                     "be rebuilt (allocates); evaluate once outside the graph capture first");
     const int rc = build_plan(b->patches, b->launch, b->plan);
     if (rc) return rc;
+    (void)own_work(b->plan, stream);   // so that the first call may be captured
     b->plan.precision = b->precision;
     for (size_t i = 0; i < b->patches.size(); ++i) b->generations[i] = b->patches[i]->generation;
     return FPHO_OK;
@@ -887,14 +934,27 @@ int evaluate_sync(fpho_patch *p, const fpho_source *prop, double **out_host) {
     const int64_t need = prop_bytes / (int64_t)sizeof(double) + plan.out.n;
     if (p->io_host.n < need) HIP_TRY(p->io_host.alloc(need));
     std::memcpy(p->io_host.ptr, prop, sizeof(fpho_source) * plan.prop.n);
-    HIP_TRY(hipMemcpyAsync(plan.prop.ptr, p->io_host.ptr, sizeof(fpho_source) * plan.prop.n,
-                           hipMemcpyHostToDevice, nullptr));
-    rc = run_plan(plan, p->status.ptr, plan.prop.ptr, plan.out.ptr,
-                  plan.out.ptr + p->n_bands, nullptr);
-    if (rc) return rc;
     *out_host = p->io_host.ptr + prop_bytes / (int64_t)sizeof(double);
-    HIP_TRY(hipMemcpyAsync(*out_host, plan.out.ptr, sizeof(double) * plan.out.n,
-                           hipMemcpyDeviceToHost, nullptr));
+    {
+        SharedWork *shared = shared_work(p->device);
+        std::lock_guard<std::mutex> lock(shared->mu);
+        const int64_t bytes = work_bytes(plan);
+        unsigned char *work = nullptr;
+        if (bytes > 0) {
+            if (shared->buf.n < bytes &&
+                shared->buf.alloc(std::max(bytes, shared->buf.n * 3 / 2)) != hipSuccess)
+                (void)hipGetLastError();   // one wave per tile
+            if (shared->buf.n >= bytes) work = shared->buf.ptr;
+        }
+        HIP_TRY(hipMemcpyAsync(plan.prop.ptr, p->io_host.ptr,
+                               sizeof(fpho_source) * plan.prop.n, hipMemcpyHostToDevice,
+                               nullptr));
+        rc = run_plan(plan, p->status.ptr, work, plan.prop.ptr, plan.out.ptr,
+                      plan.out.ptr + p->n_bands, nullptr);
+        if (rc) return rc;
+        HIP_TRY(hipMemcpyAsync(*out_host, plan.out.ptr, sizeof(double) * plan.out.n,
+                               hipMemcpyDeviceToHost, nullptr));
+    }
     HIP_TRY(hipStreamSynchronize(nullptr));
     return FPHO_OK;
 }
@@ -995,6 +1055,9 @@ int fpho_patch_create(const fpho_patch_desc *d, int return_residual, fpho_patch 
         delete p;
         return rc;
     }
+    SharedWork *shared = shared_work(p->device);
+    std::lock_guard<std::mutex> lock(shared->mu);
+    ++shared->patches;
     *out = p;
     return FPHO_OK;
 }
@@ -1093,7 +1156,10 @@ int fpho_patch_status(fpho_patch *p, uint32_t *status, int clear) {
 int fpho_patch_free(fpho_patch *p) {
     if (!p) return FPHO_OK;
     (void)hipDeviceSynchronize();
+    SharedWork *shared = shared_work(p->device);
     delete p;
+    std::lock_guard<std::mutex> lock(shared->mu);
+    if (--shared->patches == 0) shared->buf.release();
     return FPHO_OK;
 }
 
@@ -1113,8 +1179,8 @@ int fpho_evaluate_async(fpho_patch *p, const fpho_source *prop_dev, double *chi2
     if (!p || !prop_dev || !chi2_dev || !dchi2_dev) return fail(FPHO_E_ARG, "null argument");
     int rc = ensure_patch_plan(p, (hipStream_t)stream);
     if (rc) return rc;
-    return run_plan(p->plan, p->status.ptr, prop_dev, chi2_dev, dchi2_dev,
-                    (hipStream_t)stream);
+    return run_plan(p->plan, p->status.ptr, own_work(p->plan, (hipStream_t)stream), prop_dev,
+                    chi2_dev, dchi2_dev, (hipStream_t)stream);
 }
 
 int fpho_evaluate_async_noalloc(fpho_patch *p, const fpho_source *prop_dev, double *chi2_dev,
@@ -1153,7 +1219,8 @@ int fpho_evaluate_async_noalloc(fpho_patch *p, const fpho_source *prop_dev, doub
     unsigned char *base = nullptr;
     const int rc = scratch_address(device, &base);
     if (rc) return rc;
-    PlanPtrs q = plan_ptrs(plan, p->status.ptr);
+    // one wave per tile: its work buffers fit the scratch array
+    PlanPtrs q = plan_ptrs(plan, p->status.ptr, nullptr);
     q.gauss = reinterpret_cast<ImgGauss *>(base + o_gauss);
     q.gauss64 = reinterpret_cast<ImgGauss64 *>(base + o_gauss64);
     q.gboxes = reinterpret_cast<int4 *>(base + o_gboxes);
@@ -1161,8 +1228,6 @@ int fpho_evaluate_async_noalloc(fpho_patch *p, const fpho_source *prop_dev, doub
     q.cpart = reinterpret_cast<double *>(base + o_cpart);
     q.counter = reinterpret_cast<int32_t *>(base + o_counter);
     q.timing = false;
-    q.hot = nullptr;   // one wave per tile: its work buffers fit the scratch array
-    q.n_items = 0;
     return run_ptrs(q, prop_dev, chi2_dev, dchi2_dev, (hipStream_t)stream);
 }
 
@@ -1193,8 +1258,8 @@ int fpho_evaluate_response_async(fpho_patch *p, const fpho_source *prop_dev, dou
                     p->n_sources, FPHO_MAXSOURCES);
     int rc = ensure_patch_plan(p, (hipStream_t)stream);
     if (rc) return rc;
-    rc = run_plan(p->plan, p->status.ptr, prop_dev, chi2_dev, p->plan.dchi2_tmp.ptr,
-                  (hipStream_t)stream);
+    rc = run_plan(p->plan, p->status.ptr, own_work(p->plan, (hipStream_t)stream), prop_dev,
+                  chi2_dev, p->plan.dchi2_tmp.ptr, (hipStream_t)stream);
     if (rc) return rc;
     HIP_TRY(launch_response(p->plan.dchi2_tmp.ptr, p->n_bands, p->n_sources, resp_dev,
                             (hipStream_t)stream));
@@ -1269,7 +1334,8 @@ int fpho_batch_evaluate_async(fpho_batch *b, const fpho_source *props, double *c
     if (!b || !props || !chi2 || !dchi2) return fail(FPHO_E_ARG, "null argument");
     const int rc = ensure_batch_plan(b, (hipStream_t)stream);
     if (rc) return rc;
-    return run_plan(b->plan, b->plan.status.ptr, props, chi2, dchi2, (hipStream_t)stream);
+    return run_plan(b->plan, b->plan.status.ptr, own_work(b->plan, (hipStream_t)stream), props,
+                    chi2, dchi2, (hipStream_t)stream);
 }
 
 int fpho_batch_set_timing(fpho_batch *b, int on) {
@@ -1364,9 +1430,8 @@ int fpho_batch_evaluate_theta_async(fpho_batch *b, const fpho_spline *s, const d
     if (rc) return rc;
     HIP_TRY(launch_theta(b->plan.srcs.ptr, b->plan.n_srcs, theta, s->view, props,
                          b->plan.src64.ptr, b->plan.status.ptr, (hipStream_t)stream));
-    return run_plan(b->plan, b->plan.status.ptr, (const Source64 *)b->plan.src64.ptr, chi2,
-                    dchi2,
-                    (hipStream_t)stream);
+    return run_plan(b->plan, b->plan.status.ptr, own_work(b->plan, (hipStream_t)stream),
+                    (const Source64 *)b->plan.src64.ptr, chi2, dchi2, (hipStream_t)stream);
 }
 
 int fpho_batch_stack_grad_async(fpho_batch *b, const double *chi2, const double *dchi2,

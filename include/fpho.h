@@ -154,6 +154,10 @@ typedef struct fpho_launch {
     int32_t cull;             /* 1: skip (tile, Gaussian) pairs whose cutoff
                                  box misses the tile (results unchanged)    */
 } fpho_launch;
+/* Plans of up to 320 tiles per CU run their pixel pass in two launches of one
+ * wave per workgroup (each 64-pixel slot, then each tile and source), whatever
+ * waves_per_group, persistent and groups_per_cu say; results do not depend on
+ * the route. */
 
 /* ---------------------------------------------------------------- runtime */
 const char *fpho_last_error(void);
@@ -206,7 +210,9 @@ int fpho_evaluate(fpho_patch *p, const fpho_source *proposal_host,
  * [n_bands][n_sources][7].  No host synchronisation.  It allocates only
  * when the patch changed since its last evaluation (new metadata, a swap,
  * a launch or residual-write change): then its plan is rebuilt first, or,
- * if `stream` is capturing a graph, FPHO_E_STATE is returned instead.
+ * if `stream` is capturing a graph, FPHO_E_STATE is returned instead; and, for
+ * the two-launch workspace, at the first such call after synchronous ones
+ * (not while capturing: that call then runs one wave per tile).
  * Invalid proposal values set bits of the status word (fpho_patch_status). */
 int fpho_evaluate_async(fpho_patch *p, const fpho_source *proposal_dev,
                         double *chi2_dev, double *dchi2_dev, void *stream);
@@ -223,7 +229,8 @@ int fpho_evaluate_async(fpho_patch *p, const fpho_source *proposal_dev,
  * fpho_evaluate_async once, which rebuilds them; until then this returns
  * FPHO_E_STATE.  All calls on one GPU share its scratch array, so calls that
  * overlap on one GPU (on different streams or threads) race: order them on
- * one stream.  Invalid proposal values set the patch's status word. */
+ * one stream.  Invalid proposal values set the patch's status word.  It runs
+ * one wave per tile at every size (fpho_launch). */
 int fpho_evaluate_async_noalloc(fpho_patch *p, const fpho_source *proposal_dev,
                                 double *chi2_dev, double *dchi2_dev, void *stream);
 
