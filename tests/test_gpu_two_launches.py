@@ -4,6 +4,7 @@ zero-allocation entry point keeps: equal bit for bit at every tile size and
 precision mode, on exposures whose last tile, slot and Gaussian block are
 partly filled."""
 import ctypes
+from concurrent.futures import ThreadPoolExecutor
 
 import numpy as np
 import pytest
@@ -62,3 +63,68 @@ def test_two_launches_equal_one_wave_per_tile(hip, name, K):
                     assert np.all(np.isfinite(a)) and np.array_equal(a, b), (cull, mode)
     finally:
         patch.free()
+
+
+def _evaluators(patch, scene, theta):
+    nb, ns = len(patch.band_N), int(patch.n_sources)
+    prop = proposal_for(scene, synth.make_proposals(theta, nb, 1, config=61)[0])
+    prop_dev = torch.from_numpy(np.ascontiguousarray(prop, dtype=source_struct_dtype)
+                                .view(np.uint8).copy()).cuda()
+    chi2 = torch.full((nb,), 7.0, dtype=torch.float64, device="cuda")
+    dchi2 = torch.full((nb * ns * 7,), 7.0, dtype=torch.float64, device="cuda")
+
+    def stream_ordered():
+        stream = ctypes.c_void_p(int(torch.cuda.current_stream().cuda_stream))
+        _lib.check(_lib.lib().fpho_evaluate_async(patch.device_patch, _lib.dptr(prop_dev),
+                                                  _lib.dptr(chi2), _lib.dptr(dchi2), stream))
+
+    proposer = patch.get_proposer()
+    return lambda: proposer.evaluate_proposal(prop, patch)[:2], stream_ordered, chi2, dchi2
+
+
+def test_capture_after_synchronous_evaluations_only(hip):
+    # the plan has no workspace of its own then and none may be allocated
+    patch, scene, theta = synth.make_patch(SPECS["uneven"], config=61, patch_id=6,
+                                           return_residual=False, render=oracle_render)
+    patch.send_to_device()
+    try:
+        sync, stream_ordered, chi2, dchi2 = _evaluators(patch, scene, theta)
+        want = sync()
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            stream_ordered()
+        for _ in range(3):
+            chi2.fill_(7.0)
+            dchi2.fill_(7.0)
+            graph.replay()
+            torch.cuda.synchronize()
+            assert np.array_equal(chi2.cpu().numpy(), want[0])
+            assert np.array_equal(dchi2.cpu().numpy().astype(np.float32),
+                                  np.asarray(want[1]).reshape(-1))
+            assert np.array_equal(sync()[0], want[0])
+        stream_ordered()   # with a workspace of its own
+        torch.cuda.synchronize()
+        assert np.array_equal(chi2.cpu().numpy(), want[0])
+    finally:
+        patch.free()
+
+
+def test_threads_share_the_synchronous_workspace(hip):
+    patches, calls = [], []
+    try:
+        for i, name in enumerate(("padded", "uneven", "wide_psf")):
+            patch, scene, theta = synth.make_patch(SPECS[name], config=61, patch_id=i,
+                                                   return_residual=False, render=oracle_render)
+            patch.send_to_device()
+            patches.append(patch)
+            calls.append(_evaluators(patch, scene, theta)[0])
+        want = [call() for call in calls]
+        with ThreadPoolExecutor(len(calls)) as pool:
+            got = list(pool.map(lambda call: [call() for _ in range(20)], calls))
+        for w, results in zip(want, got):
+            for r in results:
+                assert np.array_equal(r[0], w[0]) and np.array_equal(r[1], w[1])
+    finally:
+        for patch in patches:
+            patch.free()
