@@ -170,7 +170,8 @@ static_assert(sizeof(ImgGauss64) == 64, "ImgGauss64 must be 64 bytes");
 // Value parameters of ImgGauss alone: what the two-launch pixel pass streams.
 struct alignas(16) HotGauss {
     float xcen, ycen, sfxx, sfyy, sfxy, hcs, ampA;
-    uint32_t tag;   // in LDS: the Gaussian's index (pass 2: and its slots)
+    uint32_t tag;   // in the workspace: kNotPlain or 0; in LDS: the Gaussian's
+                    // index (pass 2: and its slots)
 };
 static_assert(sizeof(HotGauss) == 32, "HotGauss must be 32 bytes");
 

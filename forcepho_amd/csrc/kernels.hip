@@ -166,6 +166,18 @@ __device__ __forceinline__ uint32_t make_image_gaussian(const ExpDesc &e, const 
     return flags;
 }
 
+// Whether residual_kernel may visit a Gaussian at pixels beyond its cutoff, where
+// a pair then adds an exact zero: its centre lies within kPlainCoord of the
+// exposure's origin, its F is below 1.4e6 and its amplitude finite in FP32, so
+// v' < 3e12 and h' is finite at every pixel within kMaskedCoord.  (A NaN fails.)
+constexpr double kPlainCoord = 262144.0;   // half an FP32 step below it: under 0.01 pixel
+constexpr uint32_t kNotPlain = 1;          // HotGauss::tag in the workspace
+__device__ __forceinline__ bool plain(const ImgGauss64 &g) {
+    return fabs(g.xcen) < kPlainCoord && fabs(g.ycen) < kPlainCoord &&
+           fabs(g.sfxx) < 1.0e6 && fabs(g.sfyy) < 1.0e6 && fabs(g.sfxy) < 1.0e6 &&
+           fabs(g.ampA) < 3.0e38;
+}
+
 // Workgroups (exposure, part): one wave each, its lanes stride over the
 // exposure's n_src * n_psf Gaussians in steps of gridDim.y waves.  Bound by the
 // latency of one Gaussian's FP64 chain (sincos, divisions, square roots), so
@@ -192,7 +204,8 @@ __global__ __launch_bounds__(kWave) void convert_kernel(
         out64[e.gauss_off + j] = g64;
         boxes[e.gauss_off + j] = make_int4(g.xlo, g.xhi, g.ylo, g.yhi);
         if (hot)
-            hot[e.gauss_off + j] = {g.xcen, g.ycen, g.sfxx, g.sfyy, g.sfxy, g.hcs, g.ampA, 0};
+            hot[e.gauss_off + j] = {g.xcen, g.ycen, g.sfxx, g.sfyy, g.sfxy, g.hcs, g.ampA,
+                                    plain(g64) ? 0u : kNotPlain};
     }
 }
 
@@ -800,11 +813,11 @@ __device__ __forceinline__ bool meets(float xlo, float xhi, float ylo, float yhi
     return !(fmaxf(ea, eb) < kCutScaled * fmaf(4e-6f, wide, 1.001f));
 }
 
-// The record of Gaussian i, tagged with i (two 16-byte loads).
+// The record of Gaussian i (two 16-byte loads).
 __device__ __forceinline__ HotGauss load_hot(const HotGauss *__restrict__ hot, uint32_t i) {
     const Global<float4> p = global(reinterpret_cast<const float4 *>(hot)) + 2 * i;
     const float4 a = *(const float4 *)p, b = *(const float4 *)(p + 1);
-    return {a.x, a.y, a.z, a.w, b.x, b.y, b.z, i};
+    return {a.x, a.y, a.z, a.w, b.x, b.y, b.z, __float_as_uint(b.w)};
 }
 
 // Pass 1 of one slot.  Each block of 64 Gaussians is tested at once (lane j:
@@ -816,13 +829,17 @@ __device__ __forceinline__ HotGauss load_hot(const HotGauss *__restrict__ hot, u
 // 460 to 360 us (24576 slots, 2160 Gaussians) and from 142 to 120 (8192, 720).
 // kVisits go through together: one wait for their records and one test for
 // bright terms (four small patches: 218 us a pass with four, 232 with two).
+// A block that holds a Gaussian that is not plain() goes one visit at a time,
+// as eval_tile does: such a Gaussian is tested by its cutoff box, is visited
+// only where a lane is inside its cutoff, and is bright only above its peak.
 template <int K, bool MIXED, bool CENTRE>
 __global__ __launch_bounds__(kWave) FPHO_EVAL_OCCUPANCY void residual_kernel(
     const TileDesc *__restrict__ tiles, const int32_t *__restrict__ queue,
     const ExpDesc *__restrict__ exps, const ImgGauss *__restrict__ gauss,
     const ImgGauss64 *__restrict__ gauss64, const HotGauss *__restrict__ hot,
-    const int4 *__restrict__ slot_boxes, uint64_t *__restrict__ flags,
-    double *__restrict__ resid, float *__restrict__ weight, int32_t cull) {
+    const int4 *__restrict__ gboxes, const int4 *__restrict__ slot_boxes,
+    uint64_t *__restrict__ flags, double *__restrict__ resid, float *__restrict__ weight,
+    int32_t cull) {
     constexpr int kVisits = 4;
     const int lane = threadIdx.x;
     const int wave = xcd_rotate((int)blockIdx.x, (int)gridDim.x, 29);
@@ -836,6 +853,8 @@ __global__ __launch_bounds__(kWave) FPHO_EVAL_OCCUPANCY void residual_kernel(
     // 0.01 pixel covers the FP32 rounding of the centre
     const float xlo = key_float(box.x) - 0.01f, xhi = key_float(box.y) + 0.01f;
     const float ylo = key_float(box.z) - 0.01f, yhi = key_float(box.w) + 0.01f;
+    // no Gaussian counts as plain on a slot beyond the coordinates of plain()
+    const bool far = !(fmaxf(fmaxf(-xlo, xhi), fmaxf(-ylo, yhi)) < kMaskedCoord);
     const ImgGauss *__restrict__ g = gauss + e.gauss_off;
     const ImgGauss64 *__restrict__ g64 = gauss64 + e.gauss_off;
     const int ng = e.n_src * e.n_psf;
@@ -862,8 +881,8 @@ __global__ __launch_bounds__(kWave) FPHO_EVAL_OCCUPANCY void residual_kernel(
         const float gp = cut_exp(in, ea);
         return H.ampA * gp * fmaf(vx, vx, fmaf(vy, vy, H.hcs));
     };
-    auto subtract_bright = [&](float c, const HotGauss &H) {
-        if (__builtin_amdgcn_ballot_w64(fabsf(c) > t.tmin) == 0) {
+    auto subtract_bright = [&](float c, const HotGauss &H, float tb) {
+        if (__builtin_amdgcn_ballot_w64(fabsf(c) > tb) == 0) {
             rd -= (double)c;
             return;
         }
@@ -873,7 +892,7 @@ __global__ __launch_bounds__(kWave) FPHO_EVAL_OCCUPANCY void residual_kernel(
         asm volatile("" : "+v"(xb), "+v"(yb));
         const double b = minus_value64(
             rd, g64[__builtin_amdgcn_readfirstlane(H.tag)], xb, yb);
-        rd = fabsf(c) > t.tmin ? b : rd - (double)c;
+        rd = fabsf(c) > tb ? b : rd - (double)c;
     };
 
     __shared__ HotGauss rec[kWave];
@@ -889,13 +908,18 @@ __global__ __launch_bounds__(kWave) FPHO_EVAL_OCCUPANCY void residual_kernel(
     uint64_t *__restrict__ fl = flags + t.flag + k;
     for (int base = 0; base < ng; base += kWave, fl += K) {
         const int j = base + lane;
-        const bool hit =
+        bool hit =
             j < ng && (cull == 0 || meets(xlo - h.xcen, xhi - h.xcen, ylo - h.ycen,
                                           yhi - h.ycen, h.sfxx, h.sfyy, h.sfxy));
+        const bool odd = far || h.tag != 0;
+        const bool one_by_one = __builtin_amdgcn_ballot_w64(odd) != 0;
+        if (one_by_one && odd && cull != 0 && j < ng)
+            hit = !boxed_out(1, gboxes[e.gauss_off + j], box);
         const uint64_t m = __builtin_amdgcn_ballot_w64(hit);
         const int cnt = __builtin_popcountll(m);
         const int rank = rank_in(m);
         if (hit) {
+            h.tag = j;
             rec[rank] = h;
             if (CENTRE) rec_lo[rank] = h_lo;
         }
@@ -910,8 +934,9 @@ __global__ __launch_bounds__(kWave) FPHO_EVAL_OCCUPANCY void residual_kernel(
                 : "s"(in_lanes)
                 : "scc");
         };
+        const int together = one_by_one ? 0 : cnt - cnt % kVisits;
         int n = 0;
-        for (; n + kVisits <= cnt; n += kVisits) {
+        for (; n < together; n += kVisits) {
             HotGauss H[kVisits];
             float2 L[kVisits];
             float c[kVisits], top = 0.0f;
@@ -936,7 +961,7 @@ __global__ __launch_bounds__(kWave) FPHO_EVAL_OCCUPANCY void residual_kernel(
                 for (int u = 0; u < kVisits; ++u) rd -= (double)c[u];
             } else {
 #pragma unroll
-                for (int u = 0; u < kVisits; ++u) subtract_bright(c[u], H[u]);
+                for (int u = 0; u < kVisits; ++u) subtract_bright(c[u], H[u], t.tmin);
             }
         }
         for (; n < cnt; ++n) {
@@ -944,8 +969,14 @@ __global__ __launch_bounds__(kWave) FPHO_EVAL_OCCUPANCY void residual_kernel(
             uint64_t in_lanes;
             const float c = term(H, CENTRE ? rec_lo[n] : float2{0.0f, 0.0f}, in_lanes);
             note(in_lanes);
+            float tb = t.tmin;
+            if (one_by_one) {
+                if (in_lanes == 0) continue;
+                if (MIXED && !(g[__builtin_amdgcn_readfirstlane(H.tag)].peak > t.tmin))
+                    tb = __builtin_huge_valf();
+            }
             if (MIXED)
-                subtract_bright(c, H);
+                subtract_bright(c, H, tb);
             else
                 r -= c;
         }
@@ -1421,7 +1452,8 @@ static hipError_t launch_eval_k(const EvalArgs &a, hipStream_t stream) {
     if (a.n_items > 0) {
         hipLaunchKernelGGL((residual_kernel<K, MIXED, CENTRE>), dim3((unsigned)(K * a.n_tiles)),
                            dim3(kWave), 0, stream, a.tiles, a.queue, a.exps, a.gauss, a.gauss64,
-                           a.hot, a.slot_boxes, a.flags, a.resid, a.weight, (int32_t)a.cull);
+                           a.hot, a.gboxes, a.slot_boxes, a.flags, a.resid, a.weight,
+                           (int32_t)a.cull);
         hipLaunchKernelGGL((gradient_kernel<K, MIXED, CENTRE>), dim3((unsigned)a.n_items),
                            dim3(kWave), 0, stream, a.tiles, a.items, a.exps, a.gauss, a.hot, a.flags,
                            a.resid, a.weight, a.gpart, a.cpart);
