@@ -25,6 +25,7 @@
 
 #include <algorithm>
 
+#include "cutoff.h"
 #include "fpho_internal.h"
 #include "kernels.h"
 
@@ -166,18 +167,6 @@ __device__ __forceinline__ uint32_t make_image_gaussian(const ExpDesc &e, const 
     return flags;
 }
 
-// Whether residual_kernel may visit a Gaussian at pixels beyond its cutoff, where
-// a pair then adds an exact zero: its centre lies within kPlainCoord of the
-// exposure's origin, its F is below 1.4e6 and its amplitude finite in FP32, so
-// v' < 3e12 and h' is finite at every pixel within kMaskedCoord.  (A NaN fails.)
-constexpr double kPlainCoord = 262144.0;   // half an FP32 step below it: under 0.01 pixel
-constexpr uint32_t kNotPlain = 1;          // HotGauss::tag in the workspace
-__device__ __forceinline__ bool plain(const ImgGauss64 &g) {
-    return fabs(g.xcen) < kPlainCoord && fabs(g.ycen) < kPlainCoord &&
-           fabs(g.sfxx) < 1.0e6 && fabs(g.sfyy) < 1.0e6 && fabs(g.sfxy) < 1.0e6 &&
-           fabs(g.ampA) < 3.0e38;
-}
-
 // Workgroups (exposure, part): one wave each, its lanes stride over the
 // exposure's n_src * n_psf Gaussians in steps of gridDim.y waves.  Bound by the
 // latency of one Gaussian's FP64 chain (sincos, divisions, square roots), so
@@ -205,7 +194,9 @@ __global__ __launch_bounds__(kWave) void convert_kernel(
         boxes[e.gauss_off + j] = make_int4(g.xlo, g.xhi, g.ylo, g.yhi);
         if (hot)
             hot[e.gauss_off + j] = {g.xcen, g.ycen, g.sfxx, g.sfyy, g.sfxy, g.hcs, g.ampA,
-                                    plain(g64) ? 0u : kNotPlain};
+                                    plain(g64.xcen, g64.ycen, g64.sfxx, g64.sfyy, g64.sfxy, g64.ampA)
+                                        ? 0u
+                                        : kNotPlain};
     }
 }
 
@@ -791,26 +782,6 @@ __device__ __forceinline__ int xcd_rotate(int b, int n, int turn) {
     const int local = b >> 3, row = local >> shift;
     const int xcd = (b + 3 * row) & 7;
     return (((row << 3) + xcd) << shift) + ((local + turn * row) & ((1 << shift) - 1));
-}
-
-// False only if no point of the box [xlo, xhi] x [ylo, yhi] (relative to the
-// Gaussian's centre) lies inside its cutoff ellipse E <= 36.  The smallest E
-// of a box that does not hold the centre is on an edge that faces the centre;
-// along such an edge E is a parabola with its minimum at -(Fxy / Fyy) dx (or
-// its twin).  sF is negative, so the smallest E is the largest E'.  The limit
-// is widened by 0.1% and by the FP32 error of E, 4e-6 of it per 1 / (1 -
-// rho^2), here and in pass 1; a NaN or an indefinite F counts as meeting.
-__device__ __forceinline__ bool meets(float xlo, float xhi, float ylo, float yhi, float sfxx,
-                                      float sfyy, float sfxy) {
-    const float dx = __builtin_amdgcn_fmed3f(0.0f, xlo, xhi);
-    const float dy = __builtin_amdgcn_fmed3f(0.0f, ylo, yhi);
-    const float ya = __builtin_amdgcn_fmed3f(-sfxy * __builtin_amdgcn_rcpf(sfyy) * dx, ylo, yhi);
-    const float xb = __builtin_amdgcn_fmed3f(-sfxy * __builtin_amdgcn_rcpf(sfxx) * dy, xlo, xhi);
-    const float ea = fmaf(dx, fmaf(sfxx, dx, 2.0f * sfxy * ya), sfyy * ya * ya);
-    const float eb = fmaf(dy, fmaf(sfyy, dy, 2.0f * sfxy * xb), sfxx * xb * xb);
-    const float k = sfxx * sfyy;
-    const float wide = k * __builtin_amdgcn_rcpf(fmaxf(fmaf(-sfxy, sfxy, k), 0.0f));
-    return !(fmaxf(ea, eb) < kCutScaled * fmaf(4e-6f, wide, 1.001f));
 }
 
 // The record of Gaussian i (two 16-byte loads).
