@@ -825,13 +825,24 @@ bool capturing(hipStream_t stream) {
     return st != hipStreamCaptureStatusNone;
 }
 
+// While it lives, this thread may allocate beside a capture on another stream:
+// in the default mode an allocation fails then and makes that capture invalid.
+struct RelaxedCapture {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+    ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+};
+
 // The plan's own two-launch workspace, allocated at its first stream-ordered
-// evaluation; null (one wave per tile) where it is not to be had.
+// evaluation; null (one wave per tile) where it is not to be had.  A workspace
+// too small for the plan is given back where the plan is built, so nothing is
+// freed (and waited for) here.
 unsigned char *own_work(Plan &plan, hipStream_t stream) {
     const int64_t bytes = work_bytes(plan);
     if (bytes == 0) return nullptr;
     if (plan.work.n < bytes) {
         if (capturing(stream)) return nullptr;
+        const RelaxedCapture relaxed;
         if (plan.work.alloc(bytes) != hipSuccess) {
             (void)hipGetLastError();
             return nullptr;
