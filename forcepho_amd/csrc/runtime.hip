@@ -182,6 +182,7 @@ struct Plan {
     // held by plans that are evaluated stream ordered; synchronous evaluations
     // share one per device
     DevVec<unsigned char> work;
+    bool work_refused = false;    // no memory for it since the plan was built
     int64_t n_flags = 0, n_slots = 0;
     Span<float> gpart;
     Span<double> cpart;
@@ -629,6 +630,7 @@ int build_plan(const std::vector<fpho_patch *> &patches, const fpho_launch &laun
     if (rc) return rc;
     // (the device is idle)
     if (work_bytes(plan) > plan.work.n || work_bytes(plan) < plan.work.n / 4) plan.work.release();
+    plan.work_refused = false;
     if (n_items > 0) {
         HIP_TRY(launch_list_items(plan.tiles.ptr, plan.queue.ptr, plan.exps.ptr, plan.runs.ptr,
                                   n_tiles, plan.items.ptr, nullptr));
@@ -834,17 +836,19 @@ struct RelaxedCapture {
 };
 
 // The plan's own two-launch workspace, allocated at its first stream-ordered
-// evaluation; null (one wave per tile) where it is not to be had.  A workspace
-// too small for the plan is given back where the plan is built, so nothing is
+// evaluation; null (one wave per tile) where it is not to be had.  A plan asks
+// for it once: calls in a loop on a full card neither try again each time nor
+// change their route on the way.  A workspace too small for the plan is given back where the plan is built, so nothing is
 // freed (and waited for) here.
 unsigned char *own_work(Plan &plan, hipStream_t stream) {
     const int64_t bytes = work_bytes(plan);
     if (bytes == 0) return nullptr;
     if (plan.work.n < bytes) {
-        if (capturing(stream)) return nullptr;
+        if (plan.work_refused || capturing(stream)) return nullptr;
         const RelaxedCapture relaxed;
         if (plan.work.alloc(bytes) != hipSuccess) {
             (void)hipGetLastError();
+            plan.work_refused = true;
             return nullptr;
         }
     }
@@ -854,12 +858,26 @@ unsigned char *own_work(Plan &plan, hipStream_t stream) {
 // The two-launch workspace of synchronous evaluations, which all run on the
 // null stream: one per device, at most half as large again as the largest patch
 // evaluated needs (a plan of two launches has at most 320 tiles per CU and 2^26
-// flag words: 1 GiB), freed with the device's last patch.  The lock covers a call's launches, so
-// calls of several threads follow each other on the stream.
+// flag words: 1 GiB), freed with the device's last patch.  The lock covers a
+// call's launches, so calls of several threads follow each other on the stream.
 struct SharedWork {
     std::mutex mu;
     DevVec<unsigned char> buf;
     int64_t patches = 0;
+    int64_t refused = INT64_MAX;   // bytes not to be had since a patch was last freed
+
+    // (under the lock) null where it is not to be had
+    unsigned char *get(int64_t bytes) {
+        if (buf.n < bytes && bytes < refused) {
+            const int64_t spare = std::max(bytes, buf.n + buf.n / 2);
+            if (buf.alloc(spare) != hipSuccess &&
+                (spare == bytes || buf.alloc(bytes) != hipSuccess)) {
+                (void)hipGetLastError();
+                refused = bytes;
+            }
+        }
+        return buf.n >= bytes ? buf.ptr : nullptr;
+    }
 };
 SharedWork *shared_work(int device) {
     static SharedWork *const all = new SharedWork[kScratchDevices];   // never destroyed
@@ -950,13 +968,7 @@ int evaluate_sync(fpho_patch *p, const fpho_source *prop, double **out_host) {
         SharedWork *shared = shared_work(p->device);
         std::lock_guard<std::mutex> lock(shared->mu);
         const int64_t bytes = work_bytes(plan);
-        unsigned char *work = nullptr;
-        if (bytes > 0) {
-            if (shared->buf.n < bytes &&
-                shared->buf.alloc(std::max(bytes, shared->buf.n * 3 / 2)) != hipSuccess)
-                (void)hipGetLastError();   // one wave per tile
-            if (shared->buf.n >= bytes) work = shared->buf.ptr;
-        }
+        unsigned char *work = bytes > 0 ? shared->get(bytes) : nullptr;
         HIP_TRY(hipMemcpyAsync(plan.prop.ptr, p->io_host.ptr,
                                sizeof(fpho_source) * plan.prop.n, hipMemcpyHostToDevice,
                                nullptr));
@@ -1170,6 +1182,7 @@ int fpho_patch_free(fpho_patch *p) {
     SharedWork *shared = shared_work(p->device);
     delete p;
     std::lock_guard<std::mutex> lock(shared->mu);
+    shared->refused = INT64_MAX;
     if (--shared->patches == 0) shared->buf.release();
     return FPHO_OK;
 }

@@ -212,7 +212,9 @@ int fpho_evaluate(fpho_patch *p, const fpho_source *proposal_host,
  * a launch or residual-write change): then its plan is rebuilt first, or,
  * if `stream` is capturing a graph, FPHO_E_STATE is returned instead; and, for
  * the two-launch workspace, at the first such call after synchronous ones
- * (not while capturing: that call then runs one wave per tile).
+ * (not while capturing: that call then runs one wave per tile).  Where there is
+ * no memory for the workspace, calls run one wave per tile, with the same
+ * results, until the plan is rebuilt.
  * Invalid proposal values set bits of the status word (fpho_patch_status). */
 int fpho_evaluate_async(fpho_patch *p, const fpho_source *proposal_dev,
                         double *chi2_dev, double *dchi2_dev, void *stream);
