@@ -9,6 +9,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -211,6 +212,7 @@ struct Plan {
 };
 
 struct fpho_patch {
+    std::atomic<int> holders{1};   // its handle and the batches that contain it
     int device = 0;
     int64_t npix = 0;
     int32_t n_bands = 0, n_exp = 0, n_sources = 0, n_radii = 0;
@@ -247,6 +249,7 @@ struct fpho_batch {
     fpho_launch launch = default_launch(true);
     int precision = kPrecMixed;
     Plan plan;
+    ~fpho_batch();
 };
 
 struct fpho_spline {
@@ -884,6 +887,16 @@ SharedWork *shared_work(int device) {
     return all + std::min(std::max(device, 0), kScratchDevices - 1);
 }
 
+// Called with the device idle.
+void drop_patch(fpho_patch *p) {
+    if (--p->holders > 0) return;
+    SharedWork *shared = shared_work(p->device);
+    delete p;
+    std::lock_guard<std::mutex> lock(shared->mu);
+    shared->refused = INT64_MAX;
+    if (--shared->patches == 0) shared->buf.release();
+}
+
 int ensure_patch_plan(fpho_patch *p, hipStream_t stream) {
     if (p->plan.valid && p->plan_generation == p->generation) return FPHO_OK;
     if (capturing(stream))
@@ -983,6 +996,10 @@ int evaluate_sync(fpho_patch *p, const fpho_source *prop, double **out_host) {
 }
 
 }  // namespace
+
+fpho_batch::~fpho_batch() {
+    for (fpho_patch *p : patches) drop_patch(p);
+}
 
 // =================================================================== C ABI
 extern "C" {
@@ -1179,11 +1196,7 @@ int fpho_patch_status(fpho_patch *p, uint32_t *status, int clear) {
 int fpho_patch_free(fpho_patch *p) {
     if (!p) return FPHO_OK;
     (void)hipDeviceSynchronize();
-    SharedWork *shared = shared_work(p->device);
-    delete p;
-    std::lock_guard<std::mutex> lock(shared->mu);
-    shared->refused = INT64_MAX;
-    if (--shared->patches == 0) shared->buf.release();
+    drop_patch(p);
     return FPHO_OK;
 }
 
@@ -1301,6 +1314,7 @@ int fpho_batch_create(fpho_patch *const *patches, int n, fpho_batch **out) {
             return fail(FPHO_E_ARG, "patch %d is null", i);
         }
         b->patches.push_back(patches[i]);
+        ++patches[i]->holders;
         b->generations.push_back(0);
         b->n_sources0.push_back(patches[i]->n_sources);
     }

@@ -226,7 +226,10 @@ class PatchBase:
             self.__dict__.pop(n, None)
 
     def free(self):
-        pass
+        """Release what a device mix-in holds."""
+        release = getattr(super(), "free", None)
+        if release is not None:
+            release()
 
     def build_patch(self, npix=1, n_sources=1, n_radii=1, n_bands=1, n_exp=1):
         """Allocate zeroed arrays of every field at these counts (G = 1)."""

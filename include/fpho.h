@@ -198,6 +198,8 @@ int fpho_patch_set_residual_writes(fpho_patch *p, int on);
  * ordered evaluations (FPHO_STATUS_* bits); waits for the device first.
  * The word is reset whenever the patch's plan is rebuilt. */
 int fpho_patch_status(fpho_patch *p, uint32_t *status, int clear);
+/* Waits for the device.  A patch that batches contain stays with them until the
+ * last of them is freed. */
 int fpho_patch_free(fpho_patch *p);
 
 /* Synchronous drop-in: proposal (host, n_sources entries) in, chi2[n_bands]

@@ -10,6 +10,7 @@ import pytest
 import torch
 
 from forcepho_amd import _lib, synth
+from forcepho_amd.batch import PatchBatch
 from forcepho_amd.limits import source_struct_dtype
 from forcepho_amd.synth import PatchSpec
 from helpers import oracle_render, proposal_for
@@ -106,7 +107,7 @@ synchronous_tries = five(synchronous, other)
 own_tries = five(stream_ordered, other)
 other.set_launch()                       # its plan is built anew: asked for once more
 rebuilt_tries = five(stream_ordered, other)
-_lib.lib().fpho_patch_free(patch.device_patch)   # memory came back: asked for once more
+patch.free()                             # memory came back: asked for once more
 freed_tries = five(synchronous, other)
 print("tries", synchronous_tries, own_tries, rebuilt_tries, freed_tries, flush=True)
 assert (synchronous_tries, own_tries, rebuilt_tries, freed_tries) == (1, 1, 1, 1)
@@ -115,7 +116,7 @@ other.set_launch()
 before = count.value
 five(stream_ordered, other)
 assert asked[1] in sizes[before:count.value]
-_lib.lib().fpho_patch_free(other.device_patch)
+other.free()
 print("done", flush=True)
 """
 
@@ -134,3 +135,36 @@ def test_refused_workspace_is_not_asked_for_on_each_call(hip, tmp_path):
                          text=True, timeout=100, env=dict(os.environ, PYTHONPATH=path))
     print(run.stdout, run.stderr[-3000:], flush=True)
     assert run.returncode == 0 and "done" in run.stdout
+
+
+def test_freed_and_resent_patches_give_their_memory_back(hip):
+    """``free`` of a patch class reaches its device half: sending a patch again
+    and freeing it keep no device memory, and a batch keeps the patches it was
+    made of until it is freed."""
+    spec = PatchSpec(n_sources=1, n_bands=1, n_exp_per_band=4, side=1024, n_psf=1)
+    patch, scene, theta = synth.make_patch(spec, config=63, patch_id=1)
+
+    def used():
+        torch.cuda.synchronize()
+        free, total = torch.cuda.mem_get_info()
+        return total - free
+
+    patch.send_to_device()
+    prop = proposal_for(scene, theta)
+    want = patch.get_proposer().evaluate_proposal(prop, patch)
+    one = used()
+    pixels = 4 * 4 * spec.npix_unpadded        # bytes of its four pixel arrays
+    for _ in range(5):
+        patch.send_to_device()
+        patch.get_proposer().evaluate_proposal(prop, patch)
+    assert used() - one < pixels
+
+    batch = PatchBatch([patch])
+    batch.set_proposals([prop])
+    patch.free()
+    assert patch.device_patch is None
+    batch.evaluate()
+    torch.cuda.synchronize()
+    assert np.array_equal(batch.chi2_host(0), want[0])
+    batch.free()
+    assert one - used() > pixels
