@@ -63,7 +63,7 @@ hipError_t launch_convert(const ExpDesc *exps, int64_t n_exp, int32_t max_ng,
                           uint32_t *status, hipStream_t stream);
 hipError_t launch_eval(const EvalArgs &a, hipStream_t stream);
 hipError_t launch_list_items(const TileDesc *tiles, const int32_t *queue, const ExpDesc *exps,
-                             const int4 *runs, int64_t n_tiles, int2 *items,
+                             const int4 *runs, int64_t n_tiles, int64_t n_items, int2 *items,
                              hipStream_t stream);
 hipError_t launch_response(const double *dchi2, int32_t n_bands, int32_t n_src,
                            fpho_response *out, hipStream_t stream);

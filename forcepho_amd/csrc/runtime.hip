@@ -510,10 +510,10 @@ int64_t item_runs(const HostPlan &hp, const std::vector<int32_t> &queue,
         while (end < queue.size() && hp.tiles[queue[end]].exp == exp) ++end;
         const int32_t len = (int32_t)(end - q);
         for (int32_t i = 0; i < len; ++i) runs[q + i] = make_int4((int32_t)n_items, i, len, 0);
-        n_items += (int64_t)len * (hp.exps[exp].n_src + 1);
+        n_items += (int64_t)len * hp.exps[exp].n_src;
         q = end;
     }
-    return n_items;
+    return n_items + (int64_t)queue.size();   // and chi2 of every tile
 }
 
 int64_t align256(int64_t x) { return (x + 255) & ~(int64_t)255; }
@@ -636,7 +636,7 @@ int build_plan(const std::vector<fpho_patch *> &patches, const fpho_launch &laun
     plan.work_refused = false;
     if (n_items > 0) {
         HIP_TRY(launch_list_items(plan.tiles.ptr, plan.queue.ptr, plan.exps.ptr, plan.runs.ptr,
-                                  n_tiles, plan.items.ptr, nullptr));
+                                  n_tiles, n_items, plan.items.ptr, nullptr));
         HIP_TRY(hipStreamSynchronize(nullptr));   // other streams read the list
     }
     plan.n_exp = (int64_t)hp.exps.size();
