@@ -167,7 +167,7 @@ struct alignas(16) ImgGauss64 {
 };
 static_assert(sizeof(ImgGauss64) == 64, "ImgGauss64 must be 64 bytes");
 
-// Value parameters of ImgGauss alone: what the two-launch pixel pass streams.
+// Value parameters of ImgGauss alone: what the residual launch streams.
 struct alignas(16) HotGauss {
     float xcen, ycen, sfxx, sfyy, sfxy, hcs, ampA;
     uint32_t tag;   // in the workspace: kNotPlain or 0; in LDS: the Gaussian's
