@@ -31,6 +31,7 @@ EXPORTED = [
     "fpho_evaluate_response",
     "fpho_evaluate_response_async",
     "fpho_batch_create", "fpho_batch_layout", "fpho_batch_info",
+    "fpho_batch_two_launches",
     "fpho_batch_set_launch", "fpho_batch_set_precision",
     "fpho_batch_evaluate_async", "fpho_batch_set_timing", "fpho_batch_last_timing",
     "fpho_batch_status", "fpho_batch_free",
@@ -122,6 +123,7 @@ def _declare(lib):
         "fpho_batch_create": ([ctypes.POINTER(P), c_int, ctypes.POINTER(P)], c_int),
         "fpho_batch_layout": ([P, c_i64_p, c_i64_p, c_i64_p, c_i64_p], c_int),
         "fpho_batch_info": ([P, c_i64_p, c_i64_p, c_i64_p, c_i64_p], c_int),
+        "fpho_batch_two_launches": ([P, ctypes.POINTER(ctypes.c_int32)], c_int),
         "fpho_batch_set_launch": ([P, ctypes.POINTER(Launch)], c_int),
         "fpho_batch_set_precision": ([P, c_int], c_int),
         "fpho_batch_evaluate_async": ([P, P, P, P, P], c_int),

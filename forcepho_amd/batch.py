@@ -147,6 +147,13 @@ class PatchBatch:
         return dict(n_tiles=v[0].value, n_pairs=v[1].value, npix=v[2].value,
                     n_gauss=v[3].value)
 
+    def two_launches(self):
+        """Whether the pixel pass takes the two-launch route, which heeds
+        ``pix_per_lane`` and ``cull`` only."""
+        two = ctypes.c_int32()
+        _lib.check(_lib.lib().fpho_batch_two_launches(self.handle, ctypes.byref(two)))
+        return bool(two.value)
+
     # -- data movement ------------------------------------------------------
     def set_proposals(self, proposals):
         """Copy host proposals (a list with one ``source_struct_dtype`` array

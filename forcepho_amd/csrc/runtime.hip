@@ -220,6 +220,7 @@ struct fpho_patch {
     std::vector<int16_t> band_start, band_N;
     std::vector<int32_t> exposure_start, exposure_N, n_psf_per_source, psfgauss_start;
     std::vector<float> G_host;
+    std::vector<double> reach;   // [n_exp] pixels inside the widest cutoff ellipse
     // coordinate box of every 64-pixel chunk of every exposure (chunks start
     // at the exposure start): xlo, xhi, ylo, yhi as order keys
     std::vector<int64_t> chunk_start;  // [n_exp+1] first chunk of exposure e
@@ -342,6 +343,21 @@ int upload_meta(fpho_patch *p, const fpho_patch_desc *d) {
     p->n_psf_per_source.assign(d->n_psf_per_source, d->n_psf_per_source + p->n_bands);
     p->psfgauss_start.assign(d->psfgauss_start, d->psfgauss_start + p->n_exp);
     p->G_host.assign(d->G, d->G + p->n_exp);
+    // area of the cutoff ellipse d^T F d <= 36 of a round source of the largest
+    // radius, convolved with the widest PSF component
+    const double r2 = *std::max_element(d->rad2, d->rad2 + d->n_radii);
+    p->reach.assign(p->n_exp, 1.0);
+    for (int b = 0; b < p->n_bands; ++b)
+        for (int e = p->band_start[b]; e < p->band_start[b] + p->band_N[b]; ++e) {
+            const float *D = d->D + (int64_t)4 * d->n_sources * e;
+            double psf = 0.0;
+            for (int i = 0; i < d->n_psf_per_source[b]; ++i) {
+                const fpho_psf_gauss &g = d->psfgauss[d->psfgauss_start[e] + i];
+                psf = std::max(psf, (double)g.Cxx * g.Cyy - (double)g.Cxy * g.Cxy);
+            }
+            const double det = std::fabs((double)D[0] * D[3] - (double)D[1] * D[2]);
+            p->reach[e] = std::max(1.0, 36.0 * M_PI * (r2 * det + std::sqrt(psf)));
+        }
     HIP_TRY(p->rad2.upload(d->rad2, d->n_radii));
     HIP_TRY(p->D.upload(d->D, 4 * nes));
     HIP_TRY(p->CW.upload(d->CW, 4 * nes));
@@ -364,6 +380,7 @@ struct HostPlan {
     std::vector<PatchOut> pouts;
     int64_t n_gauss = 0, n_part = 0, n_pairs = 0, npix = 0;
     int64_t n_flags = 0;  // flag words of the two-launch pixel pass
+    double beyond = 0.0;  // sum over tiles of (exposure's pixels / a source's reach) - 1
     int32_t max_ng = 0;   // most image Gaussians of one exposure
 };
 
@@ -409,6 +426,8 @@ void plan_patch(const fpho_patch *p, int K, int64_t src_base, int64_t chi2_base,
             hp.max_ng = std::max(hp.max_ng, ns * np);
             const int32_t n_e = p->exposure_N[e];
             hp.npix += n_e;
+            hp.beyond += std::max(0.0, n_e / p->reach[e] - 1.0) *
+                         ((n_e + tile_pix - 1) / tile_pix);
             hp.n_pairs += (int64_t)n_e * ns * np;
             for (int32_t off = 0; off < n_e; off += tile_pix) {
                 TileDesc t;
@@ -488,12 +507,22 @@ std::vector<int32_t> cost_order(const HostPlan &hp) {
 // counts for more (K = 8: 106394 7072 / 6639 (7288 / 7420), 146737 9119 / 9041
 // (9381 / 10056); K = 4: 110912 3476 / 3399 (3677 / 3729), 211725 7089 / 7228
 // (7607 / 8137)).
+// Exposures much wider than a source's reach have mostly (tile, source) waves with
+// nothing to do, and slots whose residuals are written and read for nothing; once
+// the tiles fill the chip that costs more than the split gives.  By the sum over
+// tiles of the exposure's area in units of the reach, less one, in wave slots (us,
+// one wave per tile / two launches, 30 and 5 sources): 1024^2 pixels of 3.7
+// reaches, 8192 tiles (2.7) 404 / 393 and 142 / 140, 16384 tiles (5.4) 368 / 406
+// and 147 / 160, 32768 (11) 927 / 1597 and 326 / 518; 512^2 of 8.2, 4096 tiles
+// (3.6) 97 / 95 (6 sources), 16384 (14) 228 / 263; 2048^2 of 15, 8192 tiles (14)
+// 174 / 350 and 95 / 128.  256^2 pixels of 0.2 reaches count nothing.
 // A plan with more than 2^26 flag words (512 MiB: thousands of Gaussians on
 // every pixel) takes one wave per tile too, so the workspace stays bounded, and
 // so does one with 2^26 (tile, source) waves, a launch's limit of 2^32 threads.
 bool two_launches(const HostPlan &hp) {
     const int64_t wave_slots = (int64_t)32 * cu_count_cached();
     return (int64_t)hp.tiles.size() <= 10 * wave_slots &&
+           hp.beyond <= 4.0 * (double)wave_slots &&
            hp.n_flags <= (int64_t)1 << 26 &&
            hp.n_part / kNParams + (int64_t)hp.tiles.size() < (int64_t)1 << 26;
 }
@@ -1347,6 +1376,12 @@ int fpho_batch_info(const fpho_batch *b, int64_t *n_tiles, int64_t *n_pairs, int
     if (n_pairs) *n_pairs = b->plan.n_pairs;
     if (npix) *npix = b->plan.npix;
     if (n_gauss) *n_gauss = b->plan.n_gauss;
+    return FPHO_OK;
+}
+
+int fpho_batch_two_launches(const fpho_batch *b, int32_t *two) {
+    if (!b || !two) return fail(FPHO_E_ARG, "null argument");
+    *two = b->plan.valid && b->plan.work.n > 0 && work_bytes(b->plan) > 0 ? 1 : 0;
     return FPHO_OK;
 }
 

@@ -156,8 +156,10 @@ typedef struct fpho_launch {
 } fpho_launch;
 /* Plans of up to 320 tiles per CU run their pixel pass in two launches of one
  * wave per workgroup (each 64-pixel slot, then each tile and source), whatever
- * waves_per_group, persistent and groups_per_cu say; results do not depend on
- * the route. */
+ * waves_per_group, persistent and groups_per_cu say, unless their exposures are
+ * many times wider than a source reaches, hold 2^26 blocks of 64 Gaussians over
+ * all slots or 2^26 pairs of tile and source, or there is no memory for the
+ * workspace; results do not depend on the route. */
 
 /* ---------------------------------------------------------------- runtime */
 const char *fpho_last_error(void);
@@ -275,6 +277,8 @@ int fpho_batch_layout(const fpho_batch *b, int64_t *src_off, int64_t *chi2_off,
                       int64_t *dchi2_off, int64_t *theta_off);
 int fpho_batch_info(const fpho_batch *b, int64_t *n_tiles, int64_t *n_pairs,
                     int64_t *npix, int64_t *n_gauss);
+/* Whether the batch's evaluations take two launches (fpho_launch). */
+int fpho_batch_two_launches(const fpho_batch *b, int32_t *two);
 int fpho_batch_set_launch(fpho_batch *b, const fpho_launch *launch);
 int fpho_batch_set_precision(fpho_batch *b, int mode);
 int fpho_batch_evaluate_async(fpho_batch *b, const fpho_source *proposals_dev,
