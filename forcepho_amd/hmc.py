@@ -214,25 +214,26 @@ class HMC:
 
     def leapfrog(self, z, p, grad, eps=None):
         """n_steps leapfrog steps from (z, p) with gradient ``grad`` at z."""
-        if eps is None:
-            eps = self.eps
+        return self._steps(z, p, grad, self.eps if eps is None else eps, self.n_steps)
+
+    def _steps(self, z, p, grad, eps, n_steps):
         post = self.post
         # a subclass's own velocity or posterior goes through the torch path
-        if self.n_steps > 0 and self.dense is None and \
+        if n_steps > 0 and self.dense is None and \
                 type(self)._velocity is HMC._velocity and \
                 isinstance(post, DevicePosterior) and \
                 post.native(z, p, grad, eps, self.inv_mass):
-            return self._leapfrog_native(z, p, grad, eps)
+            return self._steps_native(z, p, grad, eps, n_steps)
         p = p + 0.5 * eps * grad
         lnp = None
-        for i in range(self.n_steps):
+        for i in range(n_steps):
             z = z + eps * self._velocity(p)
             lnp, grad = self.post(z)
-            p = p + (eps if i < self.n_steps - 1 else 0.5 * eps) * grad
+            p = p + (eps if i < n_steps - 1 else 0.5 * eps) * grad
         return z, p, lnp, grad
 
-    def _leapfrog_native(self, z, p, grad, eps):
-        """``leapfrog`` with one step kernel between evaluations: momentum
+    def _steps_native(self, z, p, grad, eps, n_steps):
+        """``_steps`` with one step kernel between evaluations: momentum
         kick, drift and transform together (22 elementwise kernels of 4.6 us
         before).  lnp is formed at the last point only, the one it is read at."""
         post = self.post
@@ -240,7 +241,7 @@ class HMC:
         args = dict(eps=eps, inv_mass=self.inv_mass)
         p1, z1, q = new(z), new(z), new(z)
         post.step(z, 0.5, grad=grad, p=p, p_out=p1, z_out=z1, q_out=q, **args)
-        for _ in range(self.n_steps - 1):
+        for _ in range(n_steps - 1):
             _, gq = post.batch.lnlike_and_grad(q, post.splines)
             z, p, p1, z1, q = z1, p1, new(z), new(z), new(z)
             post.step(z, 1.0, grad_q=gq, p=p, p_out=p1, z_out=z1, q_out=q, **args)

@@ -82,7 +82,7 @@ class NUTS(HMC):
         return (seg(self._velocity(p_start) * r) <= 0) | (seg(self._velocity(p_end) * r) <= 0)
 
     def _leapfrog1(self, z, p, grad, eps):
-        return self.leapfrog(z, p, grad, eps)   # n_steps is 1
+        return self._steps(z, p, grad, eps, 1)
 
     def trajectory(self):
         """One NUTS transition of every chain (in place)."""
