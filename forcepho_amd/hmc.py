@@ -80,9 +80,13 @@ class DevicePosterior:
 
     def native(self, *vectors):
         """Whether the step kernel stands for the torch expressions: it reads
-        contiguous float64 parameter vectors of the batch's device, and leaves
-        no autograd graph and no forward-mode tangent."""
+        contiguous float64 parameter vectors of the batch's device (its gradient
+        among them: the batch's own buffer, unless ``lnlike_and_grad`` is
+        someone else's), and leaves no autograd graph and no forward-mode
+        tangent."""
         return isinstance(self.batch, PatchBatch) and \
+            type(self.batch).lnlike_and_grad is PatchBatch.lnlike_and_grad and \
+            "lnlike_and_grad" not in vars(self.batch) and \
             type(self).__call__ is DevicePosterior.__call__ and \
             all(isinstance(v, torch.Tensor) and v.is_cuda and v.dtype == torch.float64 and
                 v.shape == self.lower.shape and v.device == self.lower.device and
