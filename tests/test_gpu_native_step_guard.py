@@ -60,3 +60,16 @@ def test_gradients_of_an_overridden_batch(target):
     finally:
         for b in batches:
             b.free()
+
+
+def test_negated_view(target):
+    patch, *rest = target
+    batch = PatchBatch([patch])
+    try:
+        _, want = results(batch, *rest)
+        native, got = results(batch, *rest, z_of=lambda z: torch._neg_view(-z))
+        assert not native
+        for a, b in zip(got, want):
+            assert torch.equal(a, b)
+    finally:
+        batch.free()
