@@ -12,6 +12,10 @@ workgroup, then fewer workgroups per CU.  Results
 do not depend on the persistent/grid choice or on W (same tiles, same fixed
 reduction order); K changes the tiling and therefore only the rounding of
 the FP32 partial sums.
+
+A plan that takes two launches heeds K and culling only: there every K is timed
+once, with the other knobs as the cache has them, so that a small batch does not
+choose among equal launches what a large one is then run with.
 """
 
 import itertools
@@ -65,9 +69,16 @@ def tune(batch, run, cands=None, reps=3, log=None):
     candidate launch of ``batch``; return (best, table)."""
     import torch
     cands = cands or candidates("batch")
-    table = []
+    kept = load_or_default("batch")
+    table, seen = [], set()
     for c in cands:
         batch.set_launch(**c)
+        if getattr(batch, "two_launches", lambda: False)():
+            heeded = {k: c[k] for k in ("pix_per_lane", "cull") if k in c}
+            if tuple(heeded.items()) in seen:
+                continue
+            seen.add(tuple(heeded.items()))
+            c = dict(kept, **heeded)
         run()
         torch.cuda.synchronize()
         start, stop = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)

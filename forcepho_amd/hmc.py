@@ -91,7 +91,8 @@ class DevicePosterior:
             all(isinstance(v, torch.Tensor) and v.is_cuda and v.dtype == torch.float64 and
                 v.shape == self.lower.shape and v.device == self.lower.device and
                 v.is_contiguous() and not v.is_neg() and
-                not (v.requires_grad and torch.is_grad_enabled()) and unpack_dual(v).tangent is None
+                not (v.requires_grad and torch.is_grad_enabled()) and
+                unpack_dual(v).tangent is None
                 for v in (self.lower, self.range, self.log_range) + vectors)
 
     def step(self, z, kick=0.0, **vectors):
