@@ -412,9 +412,9 @@ __device__ __forceinline__ HotGauss load_record(const ImgGauss *__restrict__ g, 
 }
 
 // Evaluate one wave tile.  `tile` must be wave-uniform (an SGPR value) so
-// every descriptor load below is a scalar load.  Bound by VALU issue: a VALU
-// instruction with a scalar operand issues every 4.4 cycles here, one whose
-// operands are all vector registers every 2.6, so both passes take the value
+// every descriptor load below is a scalar load.  Bound by VALU issue: an FMA
+// with a scalar operand issues every 4.1 cycles here, one whose operands are
+// all vector registers every 3.0, so both passes take the value
 // parameters of the Gaussians they visit from LDS (64 are put there at once,
 // a visit reads its own with a broadcast) and only the epilogue's constants by
 // scalar loads.  Against scalar loads throughout: 96 patches of 228564 tiles,
@@ -754,7 +754,8 @@ __global__ __launch_bounds__(256) FPHO_EVAL_OCCUPANCY void eval_persistent_kerne
 
 // ------------------------------------------------ pixel pass in two launches
 //
-// For plans whose tiles do not fill the chip (two_launches() in runtime.hip):
+// For plans whose tiles do not fill the chip many times over, with exposures not
+// much wider than a source reaches (two_launches() in runtime.hip):
 // residual_kernel runs one wave per 64-pixel slot, gradient_kernel one wave
 // per (tile, source), so a tile's work is spread over its slots and then over
 // its sources instead of being one wave's.  A pixel's Gaussians are still
@@ -764,17 +765,23 @@ __global__ __launch_bounds__(256) FPHO_EVAL_OCCUPANCY void eval_persistent_kerne
 //
 // What bounds it: VALU issue, and on small plans the serial chain of the
 // heaviest wave.  Measured (us, one wave per tile -> two launches): 16 tiles
-// of 54 Gaussians 58 -> 28; 2048 tiles of 720 535 -> 247; 6144 tiles of 2160
-// 1440 -> 905; 611 tiles of up to 1620 (four patches) 882 -> 134.
+// of 54 Gaussians 58 -> 26; 2048 tiles of 720 535 -> 216; 6144 tiles of 2160
+// 1440 -> 895; 611 tiles of up to 1620 (four patches) 882 -> 126.
 
-// xcd_swizzle with the XCDs' chunks moved on by three from row to row: an
-// exposure is often a whole number of chunks, and without that an XCD would
-// take the same part of every exposure, its crowded middle or its empty edge.
-// Chunks of 128 waves once there are several rows of them, else of 64.
+// xcd_swizzle with the XCDs' chunks moved on from row to row: an exposure is
+// often a whole number of chunks, and without that an XCD would take the same
+// part of every exposure, its crowded middle or its empty edge.  Any odd step
+// meets all 8 XCDs; by three, 60 sources on 24 exposures of 256^2 take 947 us a
+// pass (1013 without), 13 on 90 of 256^2 942 (972).
 // turn: how far a chunk's waves turn from row to row as well.  Waves are dealt to
 // the CUs in order, so without it the same CU takes the same place of every
-// exposure (turn 29 in the residual launch of 32 exposures of 128^2, 20 sources:
-// 270 -> 249 us a pass; the gradient launch goes source by source and loses 1%).
+// exposure.  29 is odd, so that it meets all places of a chunk, and near half
+// of 64: in the residual launch 20 sources on 32 exposures of 128^2 take 240 us
+// (248 without), the 60 sources 947 (932); the gradient launch goes source by
+// source and loses 1% by it.
+// Chunks of 128 waves from 2^15 waves on, else of 64 (90 exposures 942 us, all 64
+// 951, all 128 954).  Exposures that are no whole number of chunks (97^2) gain or
+// lose under 4% by any of the three.
 __device__ __forceinline__ int xcd_rotate(int b, int n, int turn) {
     const int shift = n >= 1 << 15 ? 7 : 6;   // log2 of the chunk
     const int rows = n >> (shift + 3);
@@ -793,9 +800,9 @@ __device__ __forceinline__ HotGauss load_hot(const HotGauss *__restrict__ hot, u
 
 // Pass 1 of one slot.  Each block of 64 Gaussians is tested at once (lane j:
 // Gaussian base + j) and the records of those that meet the slot go to LDS in
-// index order, from where a visit reads its own with a broadcast.  A VALU
-// instruction with a scalar operand issues every 4.4 cycles here, one whose
-// operands are all vector registers every 2.6; 8 of a visit's 18 read the
+// index order, from where a visit reads its own with a broadcast.  An FMA
+// with a scalar operand issues every 4.1 cycles here, one whose operands are
+// all vector registers every 3.0; 8 of a visit's 18 instructions read the
 // record, so taking it from LDS instead of by scalar loads cut the kernel from
 // 460 to 360 us (24576 slots, 2160 Gaussians) and from 142 to 120 (8192, 720).
 // kVisits go through together: one wait for their records and one test for

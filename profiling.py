@@ -15,7 +15,7 @@ Usage (each ``<dir>`` is a rocprofv3 ``-d`` output directory):
 
 ``traffic`` prints the summary that ``bench.py`` reads for ``roofline.traffic``.
 It carries a digest of the kernel sources' code (``forcepho_amd/csrc/kernels.hip`` and
-the two headers it compiles with), so a summary taken on other kernel code
+the headers it compiles with), so a summary taken on other kernel code
 is recognised as stale.
 """
 
@@ -33,7 +33,7 @@ CSRC = os.path.join(HERE, "forcepho_amd", "csrc")
 KERNEL_SOURCE = os.path.join(CSRC, "kernels.hip")
 # the sources whose code fixes the pixel-pass machine code
 KERNEL_SOURCES = [KERNEL_SOURCE, os.path.join(CSRC, "kernels.h"),
-                  os.path.join(CSRC, "fpho_internal.h")]
+                  os.path.join(CSRC, "fpho_internal.h"), os.path.join(CSRC, "cutoff.h")]
 COPY_BYTES = 1 << 30   # bench.py --copy-calibration copies 1 GiB per dispatch
 
 __all__ = ["kernel_source_digest", "kernel_stats", "api_stats", "counter_medians",
@@ -49,7 +49,7 @@ def _code_only(text):
 
 def kernel_source_digest(paths=None):
     """First 16 hex digits of the SHA-256 of the kernel sources' code
-    (``kernels.hip``, ``kernels.h``, ``fpho_internal.h``; comments and
+    (``kernels.hip``, ``kernels.h``, ``fpho_internal.h``, ``cutoff.h``; comments and
     whitespace do not count, so a profile stays valid across comment edits)."""
     h = hashlib.sha256()
     for p in paths or KERNEL_SOURCES:
