@@ -832,7 +832,8 @@ __global__ __launch_bounds__(kWave) FPHO_EVAL_OCCUPANCY void residual_kernel(
     const float xlo = key_float(box.x) - 0.01f, xhi = key_float(box.y) + 0.01f;
     const float ylo = key_float(box.z) - 0.01f, yhi = key_float(box.w) + 0.01f;
     // no Gaussian counts as plain on a slot beyond the coordinates of plain()
-    const bool far = !(fmaxf(fmaxf(-xlo, xhi), fmaxf(-ylo, yhi)) < kMaskedCoord);
+    const uint64_t far = __builtin_amdgcn_ballot_w64(
+        !(fmaxf(fmaxf(-xlo, xhi), fmaxf(-ylo, yhi)) < kMaskedCoord));
     const ImgGauss *__restrict__ g = gauss + e.gauss_off;
     const ImgGauss64 *__restrict__ g64 = gauss64 + e.gauss_off;
     const int ng = e.n_src * e.n_psf;
@@ -889,10 +890,11 @@ __global__ __launch_bounds__(kWave) FPHO_EVAL_OCCUPANCY void residual_kernel(
         bool hit =
             j < ng && (cull == 0 || meets(xlo - h.xcen, xhi - h.xcen, ylo - h.ycen,
                                           yhi - h.ycen, h.sfxx, h.sfyy, h.sfxy));
-        const bool odd = far || h.tag != 0;
-        const bool one_by_one = __builtin_amdgcn_ballot_w64(odd) != 0;
-        if (one_by_one && odd && cull != 0 && j < ng)
-            hit = !boxed_out(1, gboxes[e.gauss_off + j], box);
+        const bool one_by_one = (far | __builtin_amdgcn_ballot_w64(h.tag != 0)) != 0;
+        if (one_by_one) {
+            if (cull != 0 && j < ng && (far != 0 || h.tag != 0))
+                hit = !boxed_out(1, gboxes[e.gauss_off + j], box);
+        }
         const uint64_t m = __builtin_amdgcn_ballot_w64(hit);
         const int cnt = __builtin_popcountll(m);
         const int rank = rank_in(m);
